@@ -15,8 +15,11 @@
 //   fw_prefill_pp_pair_kernel, fw_prefill_d256_pair_kernel
 //                              the same on large dense grids, two mirrored q
 //                              tiles per workgroup
-//   fw_prefill_staged_kernel   the other head dims (64, 96, 192, 384, 512 and
-//                              mixed q / v widths): K/V staged in registers
+//   fw_prefill_d64_kernel      head dims 64/64, bf16 K/V: 4 waves, three
+//                              workgroups per CU
+//   fw_prefill_staged_kernel   the other head dims (96, 192, 384, 512, mixed
+//                              q / v widths) and fp8 pools at 64: K/V staged
+//                              in registers
 // In all of them a wave owns 32 query rows, each lane one row, and computes
 //   S^T (32 keys x 32 rows) = K x Q^T        (Q^T resident in registers)
 //   online softmax in log2 units
@@ -213,7 +216,7 @@ struct KvAddr {
   }
 };
 
-// fp8 K/V and head_dim 256: 4 waves = 128 rows; K/V rows are widened to
+// The register-staged kernel: 4 waves = 128 rows; K/V rows are widened to
 // bf16 in registers and staged as
 //   Ks  [64 keys][D + 8 bf16]  row-major (row pad keeps ds_read_b128 conflict-free)
 //   Vt  [D dims][68 bf16]      transposed, keys in pairs (so the PV operand of
@@ -1818,6 +1821,324 @@ __global__ __launch_bounds__(256, 1) void fw_prefill_d256_pair_kernel(PrefillArg
   d256_body<FW_KV_DENSE, SOFTCAP, FW_BF16>(a, a.n_qt - 1 - qt, bh);
 }
 
+// ---------------------------------------------------------------------------
+// head_dim 64, bf16 K/V: workgroup = 4 waves of 32 q rows each (2^hpw_shift
+// <= 4 query heads of a GQA group over the same rows), three workgroups per
+// CU.  A 64-key tile is 16 MFMAs (512 cycles) and about as much VALU work (32
+// exponentials, 32 adds, 16 packs) a wave, so neither pipe can hide behind
+// the other inside one wave, and a single wave issues VALU at half the SIMD's
+// rate; three free-running waves per SIMD (up to 168 registers each) overlap
+// the two.  K/V tiles (8 KiB each, 128-byte rows) rotate through three LDS
+// buffers, copied straight from global memory two tiles ahead; one barrier per
+// tile.  Measured, 4 x 32/8 heads x 1999 tokens, causal: 79.8 us, 820 TFLOP/s
+// (the register-staged kernel at two waves per SIMD: 137.7 us, 476); with
+// softcap 50 91.8 (151.6) us; 8K and 16K tokens 962 and 1,025 TFLOP/s, at which
+// the chip's power sets the clock (1.96 GHz).  Four waves per SIMD spill (128
+// registers): 120 us.  Without the exponentials 66 us, without the copies 69.
+constexpr int kD6Waves = 4;
+constexpr int kD6RowB = 128;                // LDS bytes of one key row
+constexpr int kD6TileB = kKT * kD6RowB;     // 8 KiB per K or V tile
+constexpr int kD6Buf = 2 * kD6TileB;        // [K tile | V tile]
+// 16-byte chunk swizzle of a 128-byte LDS row: two rows fill the 64 banks, so
+// 16 consecutive rows need 8 distinct values over r / 2 (plain 16-byte reads),
+// and rows r and r + 2 of an aligned key quad must differ in bit 2 (the four
+// rows x four chunks that 32 lanes of a transposing read cover).
+__device__ __forceinline__ int swz64(int r) {
+  return 4 * ((r >> 1) & 1) + 2 * ((r >> 2) & 1) + ((r >> 3) & 1);
+}
+
+template <int MODE, bool SOFTCAP>
+__global__ __launch_bounds__(256, 3) void fw_prefill_d64_kernel(PrefillArgs a) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[3 * kD6Buf];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31;
+  const int g = lane >> 5;
+  // wave w: head hg * 2^hpw_shift + (w >> wph_shift), rows q0 + 32 rb ..
+  const int wph_shift = 2 - a.hpw_shift;
+  const int rb = w & ((1 << wph_shift) - 1);
+  const int R = (32 * kD6Waves) >> a.hpw_shift;
+
+  // ------------------------------------------------------------ tile decode
+  int b = 0, hg, seq = 0, q0, sq_len, sk_len, qtok0 = 0, kbase = 0;
+  if constexpr (MODE == FW_KV_DENSE) {
+    const int ng = a.H >> a.hpw_shift;
+    int qt, bh;
+    dense_item(a, blockIdx.x, a.B * ng, qt, bh);
+    b = bh / ng;
+    hg = bh % ng;
+    q0 = qt * R;
+    sq_len = a.Sq;
+    sk_len = a.Sk;
+  } else {
+    int slot;
+    sched_slot(a, slot, hg);
+    if (slot >= a.sched[0]) return;
+    seq = a.sched[1 + 2 * slot];
+    q0 = a.sched[2 + 2 * slot];
+    if (seq < 0) {  // packed padding rows: out 0, lse -inf
+      const int hp = (hg << a.hpw_shift) + (w >> wph_shift);
+      const int r0 = q0 + 32 * rb + n;
+      if (r0 < a.Sq) {
+        uint16_t *o = a.out + (size_t)hp * a.osh + (size_t)r0 * a.ost;
+        for (int d = g * 32; d < g * 32 + 32; d += 8) *(u32x4_t *)(o + d) = u32x4_t{0, 0, 0, 0};
+        if (a.lse && g == 0) a.lse[(size_t)hp * a.lsh + r0] = -INFINITY;
+      }
+      return;
+    }
+    qtok0 = a.cu_q[seq];
+    sq_len = a.cu_q[seq + 1] - qtok0;
+    if constexpr (MODE == FW_KV_VARLEN) {
+      kbase = a.cu_k[seq];
+      sk_len = a.cu_k[seq + 1] - kbase;
+    } else {
+      sk_len = a.seqused_k[seq] + (a.seqused_plus_q ? sq_len : 0);
+    }
+  }
+  const int h = (hg << a.hpw_shift) + (w >> wph_shift);  // this wave's query head
+  const int hk = h / a.G;
+  const int off = sk_len - sq_len;  // bottom-right alignment
+  auto row_hi = [&](int r) {
+    const int p = r + off;
+    return a.wr >= 0 ? min(sk_len, p + a.wr + 1) : sk_len;
+  };
+  auto row_lo = [&](int r) {
+    const int p = r + off;
+    return a.wl >= 0 ? max(0, p - a.wl) : 0;
+  };
+  const int last_row = min(q0 + R, sq_len) - 1;
+  const int wg_lo = row_lo(q0);
+  const int wg_hi = row_hi(last_row);
+  const int w_first = q0 + 32 * rb;
+  const int w_last = min(w_first + 31, sq_len - 1);
+  const bool w_any = w_first <= w_last;
+  const int w_lo = w_any ? row_lo(w_first) : 0;
+  const int w_hi = w_any ? row_hi(w_last) : 0;
+  const int qrow = q0 + 32 * rb + n;
+  const bool row_ok = qrow < sq_len;
+  const int r_lo = row_lo(qrow), r_hi = row_hi(qrow);
+  const int t_begin = wg_hi > wg_lo ? wg_lo / kKT : 0;
+  const int t_end = wg_hi > wg_lo ? (wg_hi + kKT - 1) / kKT : 0;
+  const int T = t_end - t_begin;
+
+  // ---- copies: tile j lands in buffer j % 3; this wave moves key rows 16w ..
+  // 16w + 15 of K and of V, eight rows per instruction: lane l writes
+  // physical chunk l % 8 of row 8i + l / 8, which holds logical chunk
+  // (l % 8) ^ swz64(row).  The 16 rows lie on one page (P % 16 == 0).
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(FW_LDS uint8_t *)lds;
+  uint32_t kstB, vstB;
+  const uint8_t *kbase_p = nullptr, *vbase_p = nullptr;
+  if constexpr (MODE == FW_KV_PAGED) {
+    kstB = vstB = (uint32_t)a.CH * kD6RowB;
+  } else {
+    kstB = 2u * (uint32_t)a.kst;
+    vstB = 2u * (uint32_t)a.vst;
+    kbase_p = a.k + 2 * ((size_t)b * a.ksb + (size_t)hk * a.ksh + (size_t)kbase * a.kst);
+    vbase_p = a.v + 2 * ((size_t)b * a.vsb + (size_t)hk * a.vsh + (size_t)kbase * a.vst);
+  }
+  const uint32_t lr = lane >> 3;
+  const uint32_t lch = 16u * (uint32_t)((lane & 7) ^ (4 * ((lane >> 4) & 1) + 2 * ((lane >> 5) & 1)));
+  auto dma = [&](int j, int buf) __attribute__((always_inline)) {
+    const int kmax = sk_len - 1;
+    int key0 = min((t_begin + j) * kKT + 16 * w, kmax);
+    const uint8_t *kp, *vp;
+    bool bad = false;
+    if constexpr (MODE == FW_KV_PAGED) {
+      key0 &= ~15;
+      const int page = a.table[(size_t)seq * a.max_pages + key0 / a.P];
+      bad = page < 0 || page >= a.num_pages;  // never dereferenced: reads the zero rows
+      kp = a.k + (((size_t)page * a.P + key0 % a.P) * a.CH + 2 * hk) * kD6RowB;
+      if (bad) kp = kZeroKV;
+      vp = kp + kD6RowB;
+    } else {
+      kp = kbase_p + (size_t)key0 * kstB;
+      vp = vbase_p + (size_t)key0 * vstB;
+    }
+    const uint32_t lim = bad ? 0u : (uint32_t)(kmax - key0);
+    const uint32_t ra = min(lr, lim), rc = min(lr + 8u, lim);  // rows past the last key re-read it
+    const uint32_t d = lds0 + (uint32_t)(16 * w * kD6RowB) + (uint32_t)buf * kD6Buf;
+    lds_dma16x2(kp, __umul24(ra, kstB) + lch, __umul24(rc, kstB) + (lch ^ 16u), d);
+    lds_dma16x2(vp, __umul24(ra, vstB) + lch, __umul24(rc, vstB) + (lch ^ 16u), d + kD6TileB);
+  };
+  if (T > 0) dma(0, 0);
+  if (T > 1) dma(1, 1);
+
+  // ------------------------------------------------------------ Q^T operand
+  bf16x8_t qop[4];
+  {
+    const uint16_t *qp = a.q + (size_t)b * a.qsb + (size_t)h * a.qsh +
+                         (size_t)(qtok0 + (row_ok ? qrow : 0)) * a.qst;
+    const float qs = row_ok ? q_scale_of(a) : 0.f;  // rows past the end get q = 0
+    load_q_operand<64>(a, qp, g, qs, qrow + off, qop);
+  }
+  // ---- LDS operand addressing (per-lane byte offsets within a buffer):
+  // K row 32st + n, chunk 2j + g; V rows 16u + 8r + 4g + tr_a, dims 32c +
+  // 16(G & 1) + 4 tr_b (transposing reads, as in the head_dim-128 kernel).
+  uint32_t kofs[4], vofs[2][2];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) kofs[j] = lds0 + n * kD6RowB + 16 * ((2 * j + g) ^ swz64(n));
+  const int tr_a = (lane >> 2) & 3, tr_b = lane & 3;
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int row = 8 * r + 4 * g + tr_a;
+      const int chunk = 4 * c + 2 * ((lane >> 4) & 1) + (tr_b >> 1);
+      vofs[c][r] = lds0 + kD6TileB + row * kD6RowB + 16 * (chunk ^ swz64(row)) + 8 * (tr_b & 1);
+    }
+
+  f32x16_t oacc[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) oacc[c][e] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  // the QK accumulates onto -anchor (with softcap onto 0: the anchor is
+  // subtracted after the tanh), kept as a block that only a new anchor rewrites
+  f32x16_t neg_m;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) neg_m[e] = 0.f;
+
+  auto step = [&](const int t, const auto bi) __attribute__((always_inline)) {
+    constexpr uint32_t buf = decltype(bi)::value * kD6Buf;
+    // this wave's copies of tile t are complete (tile t + 1's four may be in
+    // flight); the barrier publishes every wave's and frees tile t - 1's buffer
+    if (t + 1 < T) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (t + 2 < T) dma(t + 2, (decltype(bi)::value + 2) % 3);
+    const int kb = (t_begin + t) * kKT;
+    if (kb >= w_hi || kb + kKT <= w_lo) return;  // this wave's rows see nothing here
+    f32x16_t sacc[2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        const bf16x8_t ko = __builtin_bit_cast(
+            bf16x8_t, *(const FW_LDS u32x4_t *)(kofs[j] + buf + 32 * kD6RowB * st));
+        if (SOFTCAP && j == 0) sacc[st] = mfma32(ko, qop[j], f32x16_t{});
+        else sacc[st] = mfma32(ko, qop[j], j == 0 ? neg_m : sacc[st]);
+      }
+    // online softmax against the static anchor, as in the ping-pong kernel
+    const float m_qk = m_run == -INFINITY ? 0.f : m_run;
+    if constexpr (SOFTCAP) softcap_scores<2, 16, true>(sacc, a.softcap_log2, m_qk);
+    const bool full = kb >= row_lo(w_last) && kb + kKT <= row_hi(w_first) && kb + kKT <= sk_len;
+    bool row_has_key = true;
+    if (!full) {
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int key = kb + 32 * st + 8 * (e >> 2) + 4 * g + (e & 3);
+          sacc[st][e] = (key >= r_lo && key < r_hi) ? sacc[st][e] : -INFINITY;
+        }
+      row_has_key = max(r_lo, kb) < min(r_hi, kb + kKT);
+    }
+    bf16x8_t pop[4];
+    float psum;
+    auto exponentiate = [&](float m_use) __attribute__((always_inline)) {
+      psum = -0.f;  // x + -0 = x exactly: the first add folds away
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        u32x4_t pw;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float p0 = fast_exp2(sacc[u >> 1][8 * (u & 1) + 2 * e] - m_use);
+          const float p1 = fast_exp2(sacc[u >> 1][8 * (u & 1) + 2 * e + 1] - m_use);
+          psum += p0 + p1;
+          pw[e] = pack_bf16(p0, p1);
+        }
+        pop[u] = __builtin_bit_cast(bf16x8_t, pw);
+      }
+    };
+    exponentiate(0.f);
+    if (__any(!(psum <= kPsumTrigger) || (m_run == -INFINITY && row_has_key))) {
+      asm volatile("" ::: "memory");  // a real branch: never if-converted
+      float tmax = -INFINITY;
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, sacc[st][e]);
+      tmax = wave_max_xor(tmax, 32) + m_qk;
+      const float m_new = fmaxf(m_run, tmax);
+      const float alpha = (m_run == -INFINITY) ? 0.f : fast_exp2(m_run - m_new);
+      m_run = m_new;
+      const float m_use = m_new == -INFINITY ? 0.f : m_new;
+      exponentiate(m_use - m_qk);
+      l_run *= alpha;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) oacc[c] *= alpha;
+      if constexpr (!SOFTCAP) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) neg_m[e] = -m_use;
+      }
+    }
+    l_run += psum;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const v4i16_t p0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (FW_LDS v4i16_t *)(vofs[c][0] + buf + 16 * u * kD6RowB));
+        const v4i16_t p1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (FW_LDS v4i16_t *)(vofs[c][1] + buf + 16 * u * kD6RowB));
+        const bf16x8_t vo = __builtin_bit_cast(
+            bf16x8_t, __builtin_shufflevector(p0, p1, 0, 1, 2, 3, 4, 5, 6, 7));
+        oacc[c] = mfma32(vo, pop[u], oacc[c]);
+      }
+  };
+  for (int t = 0; t < T; t += 3) {
+    step(t, std::integral_constant<int, 0>());
+    if (t + 1 < T) step(t + 1, std::integral_constant<int, 1>());
+    if (t + 2 < T) step(t + 2, std::integral_constant<int, 2>());
+  }
+
+  // ------------------------------------------------------------ epilogue
+  l_run += __shfl_xor(l_run, 32, 64);
+  float M = m_run, Lsum = l_run, oscale = 1.f;
+  if (a.sinks) {
+    const float sk = a.sinks[h] * kLog2e;
+    if (sk != -INFINITY) {
+      const float Mn = fmaxf(M, sk);
+      const float c_old = fast_exp2(M - Mn);
+      Lsum = Lsum * c_old + fast_exp2(sk - Mn);
+      oscale = c_old;
+      M = Mn;
+    }
+  }
+  const bool any = Lsum > 0.f && l_run > 0.f;
+  const float scale = any ? oscale * v_descale_of(a) / Lsum : 0.f;
+  // O goes out as whole 128-byte rows, staged through the wave's 4 KiB of LDS
+  __syncthreads();  // every wave's LDS reads of the loop are done
+  {
+    const uint32_t wbase = lds0 + (uint32_t)w * 4096u;
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        const u32x2_t wv = {pack_bf16(oacc[c][4 * rr] * scale, oacc[c][4 * rr + 1] * scale),
+                            pack_bf16(oacc[c][4 * rr + 2] * scale, oacc[c][4 * rr + 3] * scale)};
+        *(FW_LDS u32x2_t *)(wbase + n * kD6RowB + 16 * ((4 * c + rr) ^ swz64(n)) + 8 * g) = wv;
+      }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 8 * i + (lane >> 3), cc = lane & 7;
+      const u32x4_t v = *(const FW_LDS u32x4_t *)(wbase + r * kD6RowB + 16 * (cc ^ swz64(r)));
+      const int grow = q0 + 32 * rb + r;
+      if (grow < sq_len)
+        __builtin_nontemporal_store(v, (u32x4_t *)(a.out + (size_t)b * a.osb + (size_t)h * a.osh +
+                                                   (size_t)(qtok0 + grow) * a.ost + 8 * cc));
+    }
+  }
+  if (!row_ok) return;
+  if (a.lse && g == 0) {
+    a.lse[(size_t)b * a.lsb + (size_t)h * a.lsh + qtok0 + qrow] =
+        Lsum > 0.f ? (M + __log2f(Lsum)) * kLn2 : -INFINITY;
+  }
+}
+
 // One workgroup: per-sequence q tiles from cu_seqlens_q, then padding tiles
 // for the packed rows past cu_seqlens_q[num_active] (schedule.py:617-717).
 // When there are at most kSortTiles sequence tiles they are ordered by cost,
@@ -1985,18 +2306,24 @@ static bool use_pingpong(const fw_prefill_params *p) {
          head_dim_v_of(p) == 128;
 }
 
-// log2 of the query heads per ping-pong workgroup: the largest power of two
-// up to 8 that divides the GQA group size (1 for MHA).
+static bool use_d64(const fw_prefill_params *p) {
+  return p->kv_dtype == FW_BF16 && p->head_dim == 64 && head_dim_v_of(p) == 64;
+}
+
+// log2 of the query heads per workgroup: the largest power of two that
+// divides the GQA group size (1 for MHA), up to the workgroup's waves (8 in
+// the ping-pong kernel, 4 in the head_dim-64 one); the other kernels take one.
 static int pp_head_shift(const fw_prefill_params *p) {
+  const int most = use_pingpong(p) ? 3 : use_d64(p) ? 2 : 0;
   const int G = p->nheads_k > 0 ? p->nheads / p->nheads_k : 1;
   int sh = 0;
-  while (sh < 3 && G % (2 << sh) == 0) ++sh;
+  while (sh < most && G % (2 << sh) == 0) ++sh;
   return sh;
 }
 
 // q rows per schedule slot (and per dense q tile).
 static int prefill_tile_rows(const fw_prefill_params *p) {
-  return use_pingpong(p) ? kPPRows >> pp_head_shift(p) : kQT;
+  return (use_pingpong(p) ? kPPRows : kQT) >> pp_head_shift(p);
 }
 
 }  // namespace fw
@@ -2036,8 +2363,9 @@ extern "C" size_t fw_prefill_workspace_bytes(const fw_prefill_params *p) {
 
 // Kernel choice (the host has checked the head dims): 128/128 -> the ping-pong
 // kernel, 256/256 -> the d256 kernel (fp8 pools widened as they land in LDS in
-// both), everything else (head dims 64, 96, 192, 384, 512, head_dim_v !=
-// head_dim) -> the register-staged kernel.  A head_dim_v above 256 runs as
+// both), 64/64 with bf16 K/V -> the d64 kernel, everything else (head dims 96,
+// 192, 384, 512, head_dim_v != head_dim, fp8 pools at 64) -> the
+// register-staged kernel.  A head_dim_v above 256 runs as
 // launches over chunks of v and out, which keeps O within one wave's
 // registers: 256 dims each at head dim 64, 128 each at head dims 384 and 512
 // (whose Q^T operand alone takes 96-128 registers).
@@ -2082,7 +2410,8 @@ static void launch_mode(const PrefillArgs &a, dim3 grid, int kv_dtype, int d, in
       if (a.softcap_log2 != 0.f) fw_prefill_d256_kernel<MODE, true><<<grid, 256, 0, s>>>(a);
       else fw_prefill_d256_kernel<MODE, false><<<grid, 256, 0, s>>>(a);
     } else if (d == 64 && dv == 64) {
-      launch_staged<MODE, FW_BF16, 64, 64>(a, grid, s);
+      if (a.softcap_log2 != 0.f) fw_prefill_d64_kernel<MODE, true><<<grid, 256, 0, s>>>(a);
+      else fw_prefill_d64_kernel<MODE, false><<<grid, 256, 0, s>>>(a);
     } else if constexpr (MODE == FW_KV_PAGED) {  // pools at 384 and 512: 128-dim V chunks
       if (d == 384) launch_staged<MODE, FW_BF16, 384, 128>(a, grid, s);
       else launch_staged<MODE, FW_BF16, 512, 128>(a, grid, s);
@@ -2188,8 +2517,7 @@ extern "C" int fw_prefill(const fw_prefill_params *p, fw_stream_t stream) {
   a.G = p->nheads / p->nheads_k;
   a.Sq = p->seqlen_q;
   a.Sk = p->seqlen_k;
-  const bool pingpong = use_pingpong(p);
-  a.hpw_shift = pingpong ? pp_head_shift(p) : 0;
+  a.hpw_shift = pp_head_shift(p);
   a.vdim0 = 0;
   a.split_max = 0;
   a.split_code = nullptr;

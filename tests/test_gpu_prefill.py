@@ -279,7 +279,7 @@ def test_prefill_bitwise_repeat():
 # (docs/v7x.md:49-60, 157-169).
 
 
-# Head dims of q/k and v: the d256 kernel, the register-staged kernel at 64, 96
+# Head dims of q/k and v: the d256 and d64 kernels, the register-staged kernel at 96
 # and 192 and with head_dim_v != head_dim (inputs.py:193-207); the reference's
 # compiled set (test_prefill.py:52,205-208), 384 and 512 (multiples of 128,
 # inputs.py:100-140) plus 128/256 and 256/128.  A head_dim_v above 256 runs as
@@ -308,6 +308,32 @@ def test_flash_attn_func_head_dims(d, dv, b, h, hk, sq, sk, causal, window, soft
         causal=causal, window_size=window, softcap=softcap, return_softmax_lse=True)
     torch.cuda.synchronize()
     ro, rl = A.attention_ref(q, k, v, causal=causal, window_size=window, softcap=softcap,
+                             round_scaled_q=True)
+    assert_close(out.float().cpu().numpy(), head_major(ro))
+    assert_lse(lse.cpu().numpy(), rl)
+
+
+@pytest.mark.parametrize("g", [1, 2, 4, 6])  # heads a workgroup serves: 1, 2, 4, 2
+@pytest.mark.parametrize("sq,sk,causal,window,softcap", [
+    (1, 1, True, (-1, -1), 0.0),
+    (31, 65, True, (-1, -1), 0.0),      # one key past a tile
+    (33, 63, False, (-1, -1), 0.0),
+    (129, 128, True, (-1, -1), 0.0),    # a row that sees nothing, a row past a q tile
+    (97, 193, True, (70, -1), 0.0),     # four key tiles: every buffer reused
+    (64, 450, False, (300, 5), 50.0),
+])
+def test_head_dim_64_tile_edges(g, sq, sk, causal, window, softcap):
+    announce(f"d64 g{g} sq{sq} sk{sk} causal={causal} window={window} softcap={softcap}")
+    rng = np.random.default_rng(71)
+    b, hk = 2, 2
+    h = g * hk
+    q, k, v = randn(rng, (b, sq, h, 64)), randn(rng, (b, sk, hk, 64)), randn(rng, (b, sk, hk, 64))
+    s = rng.standard_normal(h).astype(np.float32) if g == 2 else None
+    out, lse = flash_attn_func(
+        to_dev_bf16(head_major(q)), to_dev_bf16(head_major(k)), to_dev_bf16(head_major(v)),
+        causal=causal, window_size=window, softcap=softcap, return_softmax_lse=True,
+        learnable_sink=None if s is None else torch.tensor(s, device=DEV))
+    ro, rl = A.attention_ref(q, k, v, causal=causal, window_size=window, softcap=softcap, sinks=s,
                              round_scaled_q=True)
     assert_close(out.float().cpu().numpy(), head_major(ro))
     assert_lse(lse.cpu().numpy(), rl)
