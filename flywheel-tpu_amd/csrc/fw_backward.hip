@@ -7,7 +7,7 @@
 //   dp = dout v^T,  ds = p (dp - delta),  delta = rowsum(dout * out)
 //   dv += p^T dout,  dk += scale ds^T q,  dq += scale ds k
 // Here that work is split into launches, all deterministic (no atomics).
-// At head dims 128/128 and 256/256, while the bf16 (B, H, Sq, Sk) planes fit
+// At head dims 64/64, 128/128 and 256/256, while the bf16 (B, H, Sq, Sk) planes fit
 // in 8 GiB of workspace and one head's in 4 GiB (the stored path):
 //   fw_bwd_dq_store_kernel    up to four query heads of one KV head over the
 //                             same 32 query rows per workgroup; q and dout live
@@ -15,7 +15,7 @@
 //                             also forms the row statistics (delta, lse_log2;
 //                             bwd.py:685-720) and writes P and delta (at 256
 //                             also dS)
-//   fw_bwd_dkv_stored_kernel  (128/128) dv = P^T dout from the stored P, dk =
+//   fw_bwd_dkv_stored_kernel  (64/64, 128/128) dv = P^T dout from the stored P, dk =
 //                             scale dS^T q with dS = P (dout v^T - delta):
 //                             three products, no score recomputed
 //   fw_bwd_dkv_ds_kernel      (256/256) dv = P^T dout and dk = scale dS^T q
@@ -406,10 +406,13 @@ __global__ __launch_bounds__(256) void fw_bwd_reduce_kernel(BwdArgs a) {
   const int key = row - bh * a.Sk;
   const int b = bh / (uint32_t)a.Hk;
   const int hk = bh - (uint32_t)b * a.Hk;
-  // dk over dqw dims, then dv over dvw dims, 128 at a time
-  for (int cb = 0; cb < a.dqw + a.dvw; cb += 128) {
-    const bool is_k = cb < a.dqw;
-    const int w = is_k ? a.dqw : a.dvw, col = is_k ? cb : cb - a.dqw;
+  // dk over dqw dims, then dv over dvw dims, 128 at a time (at 64 the upper
+  // 8 lanes of a row have nothing to sum)
+  const int blocks_k = (a.dqw + 127) / 128, blocks = blocks_k + (a.dvw + 127) / 128;
+  for (int cb = 0; cb < blocks; ++cb) {
+    const bool is_k = cb < blocks_k;
+    const int w = is_k ? a.dqw : a.dvw, col = 128 * (is_k ? cb : cb - blocks_k);
+    if (col + 8 * c >= w) continue;
     const float *part = is_k ? a.dk_part : a.dv_part;
     float sum[8] = {};
     for (int s = 0; s < a.split; ++s) {
@@ -595,11 +598,19 @@ __global__ __launch_bounds__(256, 2) void fw_bwd_dq_kernel(BwdArgs a) {
 // fall on distinct banks, and so do the 32 lanes of a transposing read (rows
 // 4m .. 4m + 3, two adjacent chunk pairs: the pair index is XORed with
 // 2(row & 3) + bit 2 of the row).
+// At head dim 64 a row is 128 bytes, so two rows fill the banks and the
+// permutation acts on 8 chunks: 16 consecutive rows take 8 values over row /
+// 2, and rows r and r + 2 of an aligned quad differ in bit 2 (4 rows x 4
+// chunks of a transposing read).
 __device__ __forceinline__ int kv_swz(int r) { return 4 * (r & 3) + 2 * ((r >> 2) & 1) + ((r >> 3) & 1); }
+template <int D>
+__device__ __forceinline__ int row_swz(int r) {
+  return D == 64 ? 4 * ((r >> 1) & 1) + 2 * ((r >> 2) & 1) + ((r >> 3) & 1) : kv_swz(r);
+}
 
 template <bool CAUSAL, int D>
-__global__ __launch_bounds__(256, D == 128 ? 2 : 1) void fw_bwd_dq_store_kernel(BwdArgs a) {
-  // D = 128 or 256 (q, k, v and out).  At 256 the kernel also stores dS
+__global__ __launch_bounds__(256, D == 64 ? 3 : D == 128 ? 2 : 1) void fw_bwd_dq_store_kernel(BwdArgs a) {
+  // D = 64, 128 or 256 (q, k, v and out).  At 256 the kernel also stores dS
   // beside P, and runs one wave per SIMD (q, dout and dq of 32 rows take 256
   // registers).
   constexpr int kRow = 2 * D;          // bytes of one K / V row
@@ -690,14 +701,14 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void fw_bwd_dq_store_kernel(
     for (int i = 0; i < 16 / kRPI; ++i) {
       const int r = 16 * w + kRPI * i + lane / kLPR;
       const int key = min(t * kBT + r, a.Sk - 1);
-      const uint32_t ch = 16u * (uint32_t)((lane % kLPR) ^ kv_swz(r));
+      const uint32_t ch = 16u * (uint32_t)((lane % kLPR) ^ row_swz<D>(r));
       const uint32_t dst = buf + (uint32_t)kRow * (16 * wu + kRPI * i);
       lds_dma16(kg, (uint32_t)(2 * (size_t)key * a.kst) + ch, dst);
       lds_dma16(vg, (uint32_t)(2 * (size_t)key * a.vst) + ch, dst + kTile);
     }
   };
   // byte offset of (row r, 16-byte chunk c) in a K or V tile
-  auto kv_at = [](int r, int c) { return (uint32_t)(kRow * r + 16 * (c ^ kv_swz(r))); };
+  auto kv_at = [](int r, int c) { return (uint32_t)(kRow * r + 16 * (c ^ row_swz<D>(r))); };
 
   // ---- stored P: the wave's first block (key tile 0) and this lane's byte
   // offset in a block's 1 KiB chunks
@@ -858,34 +869,48 @@ __device__ __forceinline__ bf16x8_t tr_rm(uint32_t Rb, int col, int u, int lane)
 // key, so its values line up with the P operand's and dS is formed in
 // registers.  Entries of P that a tile's rows do not see (the dq kernel did
 // not write them) are zeroed by a select, on tiles that need a mask only.
+// At head dim 64 a workgroup is 4 waves = 128 keys and three share a CU: both
+// stored kernels then run three waves per SIMD, and the plane (half as much
+// matrix work per P byte as at 128) is streamed by more waves.  4 x 16/16
+// heads x 2000 tokens, causal: dq 88 us and dk / dv 95 us, where the 128
+// kernels on zero-padded operands took 123 and 140 beside 95 us of padding
+// and slicing (forward + backward 412 -> 235 us).
 constexpr int kSQ = 32;                    // query rows per item
-constexpr int kStKeys = 256;               // keys per workgroup
+// waves (32 keys each) per workgroup: 8, one workgroup per CU, at head dim
+// 128; 4, three per CU (161 registers), at 64
+template <int D> constexpr int kStWaves = D == 64 ? 4 : 8;
+template <int D> constexpr int kStKeys = 32 * kStWaves<D>;  // keys per workgroup
 // P of an item sits in LDS as 1 KiB chunks at a 1152-byte stride: the two
 // 16-lane groups of a transposing read that take chunks j and j + 1 then fall
 // on different banks.
 constexpr int kPChunk = 1152;
-constexpr int kStPB = kStKeys / 16 * kPChunk;  // 18 KiB: P of an item (16 chunks)
-constexpr int kStRB = kSQ * 128 * 2;       // 8 KiB: dout (or q) rows of an item
-constexpr int kStBuf = kStPB + 2 * kStRB + 256;  // + delta
+template <int D> constexpr int kStPB = kStKeys<D> / 16 * kPChunk;  // 18 (9) KiB: P of an item
+template <int D> constexpr int kStRB = kSQ * D * 2;  // 8 (4) KiB: dout (or q) rows of an item
+template <int D> constexpr int kStBuf = kStPB<D> + 2 * kStRB<D> + 256;  // + delta
 constexpr int kStRing = 3;
 
-// LDS byte offset of (row r, dims d .. ) of a staged 32 x 128 row tile:
-// 256-byte rows whose 16-byte chunks are permuted by kv_swz(r), so that the
-// 16 rows of a plain 16-byte read and the 4 rows of a transposing read each
-// fall on distinct banks.
+// LDS byte offset of (row r, dims d .. ) of a staged 32 x D row tile: rows of
+// 2 D bytes whose 16-byte chunks are permuted by row_swz(r), so that the 16
+// rows of a plain 16-byte read and the 4 rows of a transposing read each fall
+// on distinct banks.
+template <int D>
 __device__ __forceinline__ uint32_t st_row_off(int r, int d) {
-  return (uint32_t)(r * 256 + 16 * ((d >> 3) ^ kv_swz(r)) + 2 * (d & 7));
+  return (uint32_t)(r * 2 * D + 16 * ((d >> 3) ^ row_swz<D>(r)) + 2 * (d & 7));
 }
 
-template <bool CAUSAL>
-__global__ __launch_bounds__(512, 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[kStRing * kStBuf];
+template <bool CAUSAL, int D>
+__global__ __launch_bounds__(64 * kStWaves<D>, D == 64 ? 3 : 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
+  constexpr int kNC = D / 32;           // 32-dim blocks of dv and dk
+  constexpr int kNJ = D / 16;           // MFMA links of dP; products of dV and of dK
+  constexpr int kWaves = kStWaves<D>, kKeys = kStKeys<D>, kPB = kStPB<D>, kRB = kStRB<D>;
+  constexpr int kBuf = kStBuf<D>;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kStRing * kBuf];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(FW_LDS uint8_t *)smem;
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, n = lane & 31, g = lane >> 5;
   // blockIdx.y = key block, so that the heaviest (causal: first) key blocks
   // of every head are dispatched first
-  const int k0 = blockIdx.y * kStKeys;
+  const int k0 = blockIdx.y * kKeys;
   int z = blockIdx.x;
   const int sp = z % a.split;
   z /= a.split;
@@ -901,27 +926,28 @@ __global__ __launch_bounds__(512, 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
   const int nt = max(0, (a.Sq + kSQ - 1) / kSQ - t_begin);
   const int n_items = chunk * nt;
 
-  // ---- copies: per item, wave w moves P chunks w and w + 8 (1 KiB each: 16
-  // chunks per 256 keys), dout and q rows 4w .. 4w + 3 and (every wave, the
-  // same bytes) the 32 delta values
+  // ---- copies: per item, wave w moves P chunks w and w + kWaves (1 KiB each:
+  // one per 16 keys), dout and q rows 4w .. 4w + 3 (at D = 64, 8w .. 8w + 7)
+  // and (every wave, the same bytes) the 32 delta values
   const uint32_t wu = __builtin_amdgcn_readfirstlane(w);  // w, in a scalar register
-  const int rr = 4 * w + (lane >> 4);     // this lane's dout / q row within the item
-  const int rc = (lane & 15) ^ kv_swz(rr);  // the global chunk its LDS slot holds
+  constexpr int kRPI = 512 / D, kLPR = 64 / kRPI;  // rows per copy, lanes per row
+  const int rr = kRPI * w + lane / kLPR;  // this lane's row within the item
+  const int rc = (lane % kLPR) ^ row_swz<D>(rr);  // the global chunk its LDS slot holds
   auto issue = [&](int it) __attribute__((always_inline)) {
     const int hi = it / nt, t = t_begin + it % nt;
     const int h = hk * a.G + sp * chunk + hi;
-    const uint32_t buf = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(it % kStRing) * kStBuf);
+    const uint32_t buf = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(it % kStRing) * kBuf);
     const uint8_t *pb = sgpr_ptr((const uint8_t *)(a.ws_p + stored_block(a, b * a.H + h, t, k0 / 64) * 2048));
     const uint32_t pv = 1024u * w + 16u * lane;
     lds_dma16_nt(pb, pv, buf + kPChunk * wu);
-    lds_dma16_nt(pb, pv + 8192u, buf + kPChunk * (wu + 8));
+    lds_dma16_nt(pb, pv + 1024u * kWaves, buf + kPChunk * (wu + kWaves));
     const int q = min(t * kSQ + rr, a.Sq - 1);
     const uint8_t *ob = sgpr_ptr((const uint8_t *)(a.dout + (size_t)b * a.osb + (size_t)h * a.osh));
     const uint8_t *qb = sgpr_ptr((const uint8_t *)(a.q + (size_t)b * a.qsb + (size_t)h * a.qsh));
-    lds_dma16(ob, (uint32_t)(2 * (size_t)q * a.ost) + 16u * rc, buf + kStPB + 1024u * wu);
-    lds_dma16(qb, (uint32_t)(2 * (size_t)q * a.qst) + 16u * rc, buf + kStPB + kStRB + 1024u * wu);
+    lds_dma16(ob, (uint32_t)(2 * (size_t)q * a.ost) + 16u * rc, buf + kPB + 1024u * wu);
+    lds_dma16(qb, (uint32_t)(2 * (size_t)q * a.qst) + 16u * rc, buf + kPB + kRB + 1024u * wu);
     const uint8_t *db = sgpr_ptr((const uint8_t *)(a.delta + ((size_t)b * a.H + h) * a.Sq));
-    if (lane < 32) lds_dma4(db, 4u * (uint32_t)min(t * kSQ + lane, a.Sq - 1), buf + kStPB + 2 * kStRB);
+    if (lane < 32) lds_dma4(db, 4u * (uint32_t)min(t * kSQ + lane, a.Sq - 1), buf + kPB + 2 * kRB);
   };
   constexpr int kCopies = 5;  // copies per wave per item
 
@@ -934,10 +960,10 @@ __global__ __launch_bounds__(512, 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
   const uint32_t p_base = kPChunk * (2 * w + (grp & 1)) + 16u * (2 * (4 * g + ia) + (ib & 1)) + 8u * (ib >> 1);
   // A operands (row = dim, k = query row) from the dout (dV) and q (dK) rows:
   // row K0 + a, dims 32c + 16(grp & 1) + 4b .. + 3
-  const uint32_t do_base = kStPB, q_base = kStPB + kStRB, dl_base = kStPB + 2 * kStRB;
+  const uint32_t do_base = kPB, q_base = kPB + kRB, dl_base = kPB + 2 * kRB;
   // (row K0 + a and K0 + 8 + a differ in their chunk permutation)
   auto a_off = [&](int c, int u, int h8) {
-    return st_row_off(16 * u + 8 * h8 + 4 * g + ia, 32 * c + 16 * (grp & 1) + 4 * ib);
+    return st_row_off<D>(16 * u + 8 * h8 + 4 * g + ia, 32 * c + 16 * (grp & 1) + 4 * ib);
   };
   auto tr_pair = [&](uint32_t lo_addr, uint32_t hi_addr) {
     const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FW_LDS v4i16_t *)lo_addr);
@@ -946,16 +972,16 @@ __global__ __launch_bounds__(512, 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
   };
 
   // the V row of this lane's key (dims 16j + 8g .. + 7): dP's B operand
-  bf16x8_t vop[8];
+  bf16x8_t vop[kNJ];
   {
     const uint16_t *vp = a.v + (size_t)b * a.vsb + (size_t)hk * a.vsh + (size_t)min(key, a.Sk - 1) * a.vst;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) vop[j] = __builtin_bit_cast(bf16x8_t, ld16(vp + 16 * j + 8 * g));
+    for (int j = 0; j < kNJ; ++j) vop[j] = __builtin_bit_cast(bf16x8_t, ld16(vp + 16 * j + 8 * g));
   }
 
-  f32x16_t dv_acc[4], dk_acc[4];
+  f32x16_t dv_acc[kNC], dk_acc[kNC];
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+  for (int c = 0; c < kNC; ++c)
 #pragma unroll
     for (int e = 0; e < 16; ++e) dv_acc[c][e] = dk_acc[c][e] = 0.f;
 
@@ -964,15 +990,15 @@ __global__ __launch_bounds__(512, 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
     // this wave's copies of item it are done (the next item's may be
     // outstanding); the barrier publishes every wave's, and frees the buffer
     // of item it - 1 for item it + 2
-    if (it + 1 < n_items) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+    if (it + 1 < n_items) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kCopies) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    static_assert(kCopies == 5 && kStRing == 3, "the wait counts above assume 5 copies, 3 buffers");
+    static_assert(kStRing == 3, "the wait counts above assume 3 buffers");
     __syncthreads();
     if (it + kStRing - 1 < n_items) issue(it + kStRing - 1);
     const int t = t_begin + it % nt;
-    const uint32_t buf = lds0 + (uint32_t)(it % kStRing) * kStBuf;
+    const uint32_t buf = lds0 + (uint32_t)(it % kStRing) * kBuf;
     const int qb = t * kSQ;
-    const bool full = qb + kSQ <= a.Sq && k0 + kStKeys <= a.Sk && (!CAUSAL || qb + off >= k0 + kStKeys - 1);
+    const bool full = qb + kSQ <= a.Sq && k0 + kKeys <= a.Sk && (!CAUSAL || qb + off >= k0 + kKeys - 1);
     // P of k-step u: element e at query row qb + 16u + 4g + (e & 3) (+ 8 for e >= 4)
     u32x4_t pw[2];
 #pragma unroll
@@ -995,7 +1021,7 @@ __global__ __launch_bounds__(512, 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
       }
     }
     // dP[q][key] for the item's 32 rows (value e at query row 8(e >> 2) + 4g
-    // + (e & 3)): a chain of 8 MFMAs on one accumulator, with the 8 dV
+    // + (e & 3)): a chain of D / 16 MFMAs on one accumulator, with the D / 16 dV
     // products (which need only P) between its links
     // The operands of step j + 2 are read during step j; sched_barrier
     // fences keep that order (the scheduler would otherwise move each read
@@ -1005,10 +1031,10 @@ __global__ __launch_bounds__(512, 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
     for (int e = 0; e < 16; ++e) dp[e] = 0.f;
     auto ld_da = [&](int j) __attribute__((always_inline)) {
       return __builtin_bit_cast(
-          bf16x8_t, *(const FW_LDS u32x4_t *)(uintptr_t)(buf + do_base + st_row_off(n, 16 * j + 8 * g)));
+          bf16x8_t, *(const FW_LDS u32x4_t *)(uintptr_t)(buf + do_base + st_row_off<D>(n, 16 * j + 8 * g)));
     };
     auto ld_dv = [&](int j) __attribute__((always_inline)) {
-      const int c = j & 3, u = j >> 2;
+      const int c = j % kNC, u = j / kNC;
       return tr_pair(buf + do_base + a_off(c, u, 0), buf + do_base + a_off(c, u, 1));
     };
     bf16x8_t dar[3], dvr[3];
@@ -1018,20 +1044,20 @@ __global__ __launch_bounds__(512, 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
       dvr[j] = ld_dv(j);
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (j + 2 < 8) {
+    for (int j = 0; j < kNJ; ++j) {
+      if (j + 2 < kNJ) {
         dar[(j + 2) % 3] = ld_da(j + 2);
         dvr[(j + 2) % 3] = ld_dv(j + 2);
       }
       __builtin_amdgcn_sched_barrier(0);
       dp = mfma32(dar[j % 3], vop[j], dp);
-      const int c = j & 3, u = j >> 2;
+      const int c = j % kNC, u = j / kNC;
       dv_acc[c] = mfma32(dvr[j % 3], __builtin_bit_cast(bf16x8_t, pw[u]), dv_acc[c]);
       __builtin_amdgcn_sched_barrier(0);
     }
     // the dK operands (q rows) of the first two steps, before dS is formed
     auto ld_q = [&](int i) __attribute__((always_inline)) {
-      const int u = i >> 2, c = i & 3;
+      const int u = i / kNC, c = i % kNC;
       return tr_pair(buf + q_base + a_off(c, u, 0), buf + q_base + a_off(c, u, 1));
     };
     bf16x8_t qr[3];
@@ -1054,10 +1080,10 @@ __global__ __launch_bounds__(512, 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
       sop[u] = __builtin_bit_cast(bf16x8_t, sw);
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (i + 2 < 8) qr[(i + 2) % 3] = ld_q(i + 2);
+    for (int i = 0; i < kNJ; ++i) {
+      if (i + 2 < kNJ) qr[(i + 2) % 3] = ld_q(i + 2);
       __builtin_amdgcn_sched_barrier(0);
-      dk_acc[i & 3] = mfma32(qr[i % 3], sop[i >> 2], dk_acc[i & 3]);
+      dk_acc[i % kNC] = mfma32(qr[i % 3], sop[i / kNC], dk_acc[i % kNC]);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -1069,7 +1095,7 @@ __global__ __launch_bounds__(512, 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
     uint16_t *kp = a.dk + (size_t)b * a.ksb + (size_t)hk * a.ksh + (size_t)key * a.kst;
     uint16_t *vp = a.dv + (size_t)b * a.vsb + (size_t)hk * a.vsh + (size_t)key * a.vst;
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < kNC; ++c)
 #pragma unroll
       for (int r4 = 0; r4 < 4; ++r4) {
         const f32x16_t &K = dk_acc[c], &V = dv_acc[c];
@@ -1079,9 +1105,9 @@ __global__ __launch_bounds__(512, 1) void fw_bwd_dkv_stored_kernel(BwdArgs a) {
         *(u32x2_t *)(vp + d) = u32x2_t{pack_bf16(V[4 * r4], V[4 * r4 + 1]), pack_bf16(V[4 * r4 + 2], V[4 * r4 + 3])};
       }
   } else {
-    const size_t row = ((((size_t)sp * a.B + b) * a.Hk + hk) * a.Sk + key) * 128;
+    const size_t row = ((((size_t)sp * a.B + b) * a.Hk + hk) * a.Sk + key) * D;
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < kNC; ++c)
 #pragma unroll
       for (int r4 = 0; r4 < 4; ++r4) {
         const int d = 32 * c + 8 * r4 + 4 * g;
@@ -1689,7 +1715,7 @@ int head_dim_v_of(const fw_attn_bwd_params *p) { return p->head_dim_v > 0 ? p->h
 
 // dk / dv chunks of 128 dims one dk/dv launch runs as separate workgroups
 int dkv_chunks(const fw_attn_bwd_params *p) {
-  if (p->head_dim == 128 && head_dim_v_of(p) == 128) return 1;
+  if (p->head_dim <= 128 && head_dim_v_of(p) <= 128) return 1;
   return std::max(p->head_dim, head_dim_v_of(p)) / 128;
 }
 
@@ -1709,7 +1735,7 @@ int pick_split(const fw_attn_bwd_params *p, long target) {
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// The stored path (head dims 128/128 and 256/256): the dq kernel writes P
+// The stored path (head dims 64/64, 128/128 and 256/256): the dq kernel writes P
 // (and at 256, dS) once and the dk / dv kernel reads it instead of
 // recomputing the scores.  Each plane is bf16 (B, H, Sq rounded up to 128, Sk
 // rounded up to 256) of workspace; above kStoredMaxBytes in all, or with one
@@ -1732,7 +1758,7 @@ int stored_planes(const fw_attn_bwd_params *p) { return p->head_dim == 256 ? 2 :
 
 bool use_stored(const fw_attn_bwd_params *p) {
   const int dvw = head_dim_v_of(p);
-  if (!((p->head_dim == 128 && dvw == 128) || (p->head_dim == 256 && dvw == 256))) return false;
+  if (p->head_dim != dvw || !(dvw == 64 || dvw == 128 || dvw == 256)) return false;
   const char *e = getenv("FW_BWD_STORED");
   if (e && e[0] == '0') return false;
   return head_plane_bytes(p) < ((size_t)1 << 32) &&
@@ -1757,7 +1783,7 @@ int bwd_split(const fw_attn_bwd_params *p) {
     }
     return split;
   }
-  return pick_split(p, use_stored(p) ? 1024 : 512);
+  return pick_split(p, use_stored(p) ? 1024 : 512);  // 64/64 and 128/128
 }
 
 }  // namespace
@@ -1793,6 +1819,8 @@ static void launch_wide(const BwdArgs &a, int dq_w, int dv_w, dim3 gkv, dim3 gq,
   else run(I256(), I256());
 }
 
+static int attn_bwd(const fw_attn_bwd_params *p, hipStream_t s);
+
 extern "C" int fw_attn_bwd(const fw_attn_bwd_params *p, fw_stream_t stream) {
   const int dvw = head_dim_v_of(p);
   FW_REQUIRE((p->head_dim == 128 && (dvw == 128 || dvw == 256 || dvw == 512)) ||
@@ -1801,6 +1829,25 @@ extern "C" int fw_attn_bwd(const fw_attn_bwd_params *p, fw_stream_t stream) {
              "the gfx950 backward takes head_dim / head_dim_v 128/128, 128/256, 128/512, 256/128"
              " or 256/256 (smaller head dims zero-padded to those); got %d/%d",
              p->head_dim, dvw);
+  return attn_bwd(p, (hipStream_t)stream);
+}
+
+extern "C" size_t fw_attn_bwd_d64_workspace_bytes(const fw_attn_bwd_params *p) {
+  if (p->head_dim != 64 || head_dim_v_of(p) != 64 || !use_stored(p)) return 0;
+  return fw_attn_bwd_workspace_bytes(p);
+}
+
+extern "C" int fw_attn_bwd_d64(const fw_attn_bwd_params *p, fw_stream_t stream) {
+  FW_REQUIRE(p->head_dim == 64 && head_dim_v_of(p) == 64, FW_ERR_NOT_IMPLEMENTED,
+             "fw_attn_bwd_d64 takes head_dim / head_dim_v 64/64; got %d/%d", p->head_dim,
+             head_dim_v_of(p));
+  FW_REQUIRE(use_stored(p), FW_ERR_NOT_IMPLEMENTED,
+             "fw_attn_bwd_d64 has no recomputing kernel for planes above the stored path's limits");
+  return attn_bwd(p, (hipStream_t)stream);
+}
+
+static int attn_bwd(const fw_attn_bwd_params *p, hipStream_t s) {
+  const int dvw = head_dim_v_of(p);
   FW_REQUIRE(p->nheads_k > 0 && p->nheads % p->nheads_k == 0, FW_ERR_VALUE,
              "nheads (%d) must be a multiple of nheads_k (%d)", p->nheads, p->nheads_k);
   FW_REQUIRE(p->batch > 0 && p->seqlen_q > 0 && p->seqlen_k > 0, FW_ERR_VALUE,
@@ -1873,7 +1920,6 @@ extern "C" int fw_attn_bwd(const fw_attn_bwd_params *p, fw_stream_t stream) {
   a.Sk = p->seqlen_k;
   a.scale = p->softmax_scale;
   a.qscale = p->softmax_scale * kLog2e;
-  hipStream_t s = (hipStream_t)stream;
 
   int st = FW_OK;
   if (!stored) {
@@ -1891,10 +1937,13 @@ extern "C" int fw_attn_bwd(const fw_attn_bwd_params *p, fw_stream_t stream) {
     // dq first (it writes P and dS), then dk / dv from them
     a.dq_hpw = a.G % 4 == 0 ? 4 : a.G % 2 == 0 ? 2 : 1;
     const dim3 gqs(ceil_div(p->seqlen_q, 32 * (4 / a.dq_hpw)) * (p->batch * p->nheads / a.dq_hpw));
-    const bool d256 = p->head_dim == 256;
+    const bool d256 = p->head_dim == 256, d64 = p->head_dim == 64;
     if (d256) {
       if (p->causal) fw_bwd_dq_store_kernel<true, 256><<<gqs, 256, 0, s>>>(a);
       else fw_bwd_dq_store_kernel<false, 256><<<gqs, 256, 0, s>>>(a);
+    } else if (d64) {
+      if (p->causal) fw_bwd_dq_store_kernel<true, 64><<<gqs, 256, 0, s>>>(a);
+      else fw_bwd_dq_store_kernel<false, 64><<<gqs, 256, 0, s>>>(a);
     } else {
       if (p->causal) fw_bwd_dq_store_kernel<true, 128><<<gqs, 256, 0, s>>>(a);
       else fw_bwd_dq_store_kernel<false, 128><<<gqs, 256, 0, s>>>(a);
@@ -1906,9 +1955,12 @@ extern "C" int fw_attn_bwd(const fw_attn_bwd_params *p, fw_stream_t stream) {
       if (p->causal) fw_bwd_dkv_ds_kernel<true><<<gds, 256, 0, s>>>(a);
       else fw_bwd_dkv_ds_kernel<false><<<gds, 256, 0, s>>>(a);
     } else {
-      const dim3 gst(p->batch * p->nheads_k * a.split, ceil_div(p->seqlen_k, kStKeys));
-      if (p->causal) fw_bwd_dkv_stored_kernel<true><<<gst, 512, 0, s>>>(a);
-      else fw_bwd_dkv_stored_kernel<false><<<gst, 512, 0, s>>>(a);
+      const dim3 gst(p->batch * p->nheads_k * a.split,
+                     ceil_div(p->seqlen_k, d64 ? kStKeys<64> : kStKeys<128>));
+      if (d64 && p->causal) fw_bwd_dkv_stored_kernel<true, 64><<<gst, 256, 0, s>>>(a);
+      else if (d64) fw_bwd_dkv_stored_kernel<false, 64><<<gst, 256, 0, s>>>(a);
+      else if (p->causal) fw_bwd_dkv_stored_kernel<true, 128><<<gst, 512, 0, s>>>(a);
+      else fw_bwd_dkv_stored_kernel<false, 128><<<gst, 512, 0, s>>>(a);
     }
     st = check_launch("fw_bwd_dkv_stored_kernel");
     if (st != FW_OK || a.split == 1) return st;

@@ -119,6 +119,8 @@ SIGNATURES = {
     "fw_clock_probe": (ctypes.c_int, [_c_p, _i32, _i32, _c_p]),
     "fw_attn_bwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnBwdParams)]),
     "fw_attn_bwd": (ctypes.c_int, [ctypes.POINTER(AttnBwdParams), _c_p]),
+    "fw_attn_bwd_d64_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnBwdParams)]),
+    "fw_attn_bwd_d64": (ctypes.c_int, [ctypes.POINTER(AttnBwdParams), _c_p]),
 }
 
 

@@ -5,10 +5,11 @@ autograd.py:27-109): the dense MHA / GQA / MQA forward with a causal or full
 mask has a backward (flash_attn_bwd, kernels/bwd.py:463); every other
 configuration runs its forward and raises NotImplementedError, naming the
 feature, only when a gradient is requested.  The kernels take head dims
-128/128, 128/256, 128/512, 256/128 and 256/256 (q and k / v and out); the
-reference's other backward pairs (64/64, 64/256, 64/512, 96/96, 192/128,
-192/192, test_prefill.py:205-208,285-333) run through them on zero-padded
-operands (attn_bwd_padded).  lse carries no gradient of its own.
+64/64, 128/128, 128/256, 128/512, 256/128 and 256/256 (q and k / v and out);
+the reference's other backward pairs (64/256, 64/512, 96/96, 192/128,
+192/192, test_prefill.py:205-208,285-333), and 64/64 beyond the stored path's
+plane limits, run through them on zero-padded operands (attn_bwd_padded).  lse
+carries no gradient of its own.
 """
 
 import torch
@@ -29,9 +30,19 @@ def bwd_widths(d, dv):
 def attn_bwd(q, k, v, out, dout, lse, *, qs, ks, vs, os_, ls, batch, nheads, nheads_k,
              seqlen_q, seqlen_k, softmax_scale, causal, head_dim=128, head_dim_v=None):
     """fw_attn_bwd: (dq, dk, dv) laid out like q, k, v (all contiguous), at
-    head dims the kernels take (128/128, 128/256, 128/512, 256/128, 256/256)."""
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    head dims the kernels take (128/128, 128/256, 128/512, 256/128, 256/256);
+    at 64/64 fw_attn_bwd_d64, or None when its planes exceed the limits."""
+    lib = N.lib()
+    size, launch = ((lib.fw_attn_bwd_d64_workspace_bytes, lib.fw_attn_bwd_d64)
+                    if head_dim == 64 else (lib.fw_attn_bwd_workspace_bytes, lib.fw_attn_bwd))
     p = N.AttnBwdParams()
+    p.batch, p.nheads, p.nheads_k = batch, nheads, nheads_k
+    p.head_dim, p.head_dim_v = head_dim, head_dim if head_dim_v is None else head_dim_v
+    p.seqlen_q, p.seqlen_k = seqlen_q, seqlen_k
+    nbytes = size(p)
+    if head_dim == 64 and nbytes == 0:
+        return None
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     p.q, p.k, p.v, p.out, p.dout, p.lse = (N.ptr(t) for t in (q, k, v, out, dout, lse))
     p.dq, p.dk, p.dv = N.ptr(dq), N.ptr(dk), N.ptr(dv)
     p.q_stride_b, p.q_stride_h, p.q_stride_t = qs
@@ -39,15 +50,10 @@ def attn_bwd(q, k, v, out, dout, lse, *, qs, ks, vs, os_, ls, batch, nheads, nhe
     p.v_stride_b, p.v_stride_h, p.v_stride_t = vs
     p.o_stride_b, p.o_stride_h, p.o_stride_t = os_
     p.lse_stride_b, p.lse_stride_h = ls
-    p.batch, p.nheads, p.nheads_k = batch, nheads, nheads_k
-    p.head_dim, p.head_dim_v = head_dim, head_dim if head_dim_v is None else head_dim_v
-    p.seqlen_q, p.seqlen_k = seqlen_q, seqlen_k
     p.softmax_scale, p.causal = softmax_scale, int(causal)
-    lib = N.lib()
-    nbytes = lib.fw_attn_bwd_workspace_bytes(p)
     ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=q.device)
     p.workspace, p.workspace_bytes = N.ptr(ws), ws.numel()
-    N.check(lib.fw_attn_bwd(p, N.stream_of(q)))
+    N.check(launch(p, N.stream_of(q)))
     return dq, dk, dv
 
 
@@ -59,8 +65,8 @@ def _pad_heads(x, d, width):
 
 def attn_bwd_padded(q, k, v, out, dout, lse, *, head_dim, head_dim_v, qs, ks, vs, os_,
                     **geometry):
-    """The backward at head dims the kernels do not take directly (64, 96,
-    192, and head_dim_v 64 .. 512) through the next kernel widths
+    """The backward at head dims the kernels do not take directly (64 with
+    another head_dim_v, 96, 192, and head_dim_v 64 .. 512) through the next kernel widths
     (bwd_widths): every d-vector of q and k is zero-padded to head_dim's width
     and every dv-vector of v, out and dout to head_dim_v's.  The scores, the
     softmax (the scale stays the caller's) and rowsum(dout * out) are unchanged
@@ -100,11 +106,12 @@ class FlashAttnFunction(torch.autograd.Function):
         q, k, v, out, lse = ctx.saved_tensors
         g = dict(spec["geometry"])
         d, dv = g["head_dim"], g["head_dim_v"]
-        if bwd_widths(d, dv) == (d, dv):
-            dq, dk, dv_ = attn_bwd(q, k, v, out, dout.contiguous(), lse, **g)
-        else:
-            dq, dk, dv_ = attn_bwd_padded(q, k, v, out, dout.contiguous(), lse, **g)
-        return dq, dk, dv_, None
+        dout, grads = dout.contiguous(), None
+        if (d, dv) == (64, 64) or bwd_widths(d, dv) == (d, dv):
+            grads = attn_bwd(q, k, v, out, dout, lse, **g)
+        if grads is None:
+            grads = attn_bwd_padded(q, k, v, out, dout, lse, **g)
+        return (*grads, None)
 
 
 class ForwardOnlyFunction(torch.autograd.Function):

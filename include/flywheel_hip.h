@@ -295,6 +295,12 @@ typedef struct fw_attn_bwd_params {
 
 size_t fw_attn_bwd_workspace_bytes(const fw_attn_bwd_params *p);
 int fw_attn_bwd(const fw_attn_bwd_params *p, fw_stream_t stream);
+/* The same at head_dim / head_dim_v 64/64, through the bf16 P plane only: the
+ * size is 0 (and the call FW_ERR_NOT_IMPLEMENTED) when the plane exceeds the
+ * limits above or FW_BWD_STORED=0; such calls run fw_attn_bwd on operands
+ * zero-padded to 128/128. */
+size_t fw_attn_bwd_d64_workspace_bytes(const fw_attn_bwd_params *p);
+int fw_attn_bwd_d64(const fw_attn_bwd_params *p, fw_stream_t stream);
 
 /*
  * RoPE on bf16 rows at their prefill positions, in f32 with one rounding to

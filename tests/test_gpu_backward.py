@@ -147,6 +147,24 @@ def test_backward_small_head_dims(d, b, h, hk, sq, sk, causal):
     check_grads(run(q, k, v, do, causal), q, k, v, do, causal, what)
 
 
+@pytest.mark.parametrize("stored", ["1", "0"])  # "0": zero-padded recomputing kernels
+@pytest.mark.parametrize("b,h,hk,sq,sk,causal", [
+    (1, 2, 2, 1, 1, True),
+    (2, 4, 2, 33, 129, True),      # a row past a 32-row item, a key past a 128-key block
+    (1, 4, 1, 257, 127, True),     # leading rows see no key
+    (1, 3, 1, 96, 65, False),
+    (1, 16, 1, 260, 385, True),    # query heads of a KV head split over workgroups
+])
+def test_backward_d64_edges(b, h, hk, sq, sk, causal, stored, monkeypatch):
+    monkeypatch.setenv("FW_BWD_STORED", stored)
+    what = f"bwd d64 b{b} h{h}/{hk} sq{sq} sk{sk} causal={causal} stored={stored}"
+    announce(what)
+    rng = np.random.default_rng(63)
+    q, k, v = randn(rng, (b, sq, h, 64)), randn(rng, (b, sk, hk, 64)), randn(rng, (b, sk, hk, 64))
+    do = randn(rng, (b, sq, h, 64))
+    check_grads(run(q, k, v, do, causal), q, k, v, do, causal, what)
+
+
 def test_backward_token_major_d64():
     """The reference's paired token-major d64 form (MHA, even head count)."""
     announce("bwd token-major d64")
