@@ -590,37 +590,54 @@ struct CombineArgs {
   float *lse;
   float v_descale;
   const float *vd;  // device v_descale scalar, or null (v_descale above)
+  int rows_blk;     // rows of a q tile per block
+  int groups;       // segment groups per row (threads: 16 * rows_blk * groups)
 };
 
-// One block per (work item, b), 16 threads per row of the q tile: thread t
-// merges row t / 16 over all of the row's segments, in segment order, for
-// dims 8 * (t % 16) .. + 7 (and + 128 for d256).  The loads of up to kBatch
-// segments are issued before any of them is used, so a row with at most
-// kBatch segments costs one memory latency after the range lookup.
+// A merge block's most threads: with the groups' partial results in LDS (8 VH
+// + 2 floats a thread) 1,024 take 40 KiB at d128, 512 take 36 KiB at d256.
+template <int D> constexpr int kMergeThreads = D > 128 ? 512 : 1024;
+
+// One block per (work item, rows_blk of its rows, b), 16 threads per row and
+// segment group: a group merges a contiguous run of the row's segments, in
+// segment order, thread t of it for dims 8 * (t % 16) .. + 7 (and + 128 for
+// d256); group 0 then merges the groups' results from LDS in order (so
+// repeated calls give the same bits).  The loads of up to kBatch segments are
+// issued before any of them is used, so a group costs one memory latency per
+// kBatch segments after the range lookup.
 template <int D>
-__global__ __launch_bounds__(256) void fw_decode_combine(CombineArgs c) {
+__global__ __launch_bounds__(kMergeThreads<D>) void fw_decode_combine(CombineArgs c) {
   constexpr int VH = kVH<D>;
+  extern __shared__ __attribute__((aligned(16))) uint8_t merge_lds[];
   const int part = threadIdx.x & 15;
   const bool dims_ok = 8 * part < D;  // head_dim 64: parts 8-15 hold no dims
   const DecodeArgs &a = c.d;
-  const int item = blockIdx.x;
+  const int row_blks = (a.rows_item + c.rows_blk - 1) / c.rows_blk;
+  const int item = blockIdx.x / row_blks;
   const int h = item / a.n_qtiles;
   const int qt = item % a.n_qtiles;
   const int b = blockIdx.y;
-  const int row = threadIdx.x >> 4;  // row inside the q tile
+  const int grp = (threadIdx.x >> 4) / c.rows_blk;
+  const int row = blockIdx.x % row_blks * c.rows_blk + (threadIdx.x >> 4) % c.rows_blk;
   const int r = qt * 16 + row;
-  if (row >= a.rows_item || r >= a.Rq) return;
+  const bool row_ok = row < a.rows_item && r < a.Rq;
+  if (!row_ok && c.groups == 1) return;
   const int nact = active_rows(a);
   const bool active = b < nact;
   // This row's segments, as the decode launch recorded them.
   int nsp = 0, x_first = 0;
-  if (active) {
+  if (active && row_ok) {
     int base;
     if (row_tiles(a, b, nact, base) > 0) {
       const int2 rs = a.ws_rows[b];
       x_first = rs.x;
       nsp = rs.y;
     }
+  }
+  if (c.groups > 1) {  // this group's run of segments
+    const int per = (nsp + c.groups - 1) / c.groups, first = min(nsp, grp * per);
+    nsp = min(per, nsp - first);
+    x_first += first;
   }
   const int n_items = a.Hk * a.n_qtiles;
   float M = -INFINITY, Lsum = 0.f;
@@ -653,6 +670,34 @@ __global__ __launch_bounds__(256) void fw_decode_combine(CombineArgs c) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[4 * q4 + e] = acc[4 * q4 + e] * c_old + v[i][q4][e] * c_new;
       Lsum = Lsum * c_old + ml[i].y * c_new;
+      M = Mn;
+    }
+  }
+  if (c.groups > 1) {
+    const int tpg = 16 * c.rows_blk, t = threadIdx.x % tpg;  // threads of a group, index in it
+    f32x4_t *lds_o = (f32x4_t *)merge_lds;  // [group][chunk][t]
+    float2 *lds_ml = (float2 *)(merge_lds + (size_t)c.groups * tpg * 8 * VH * sizeof(float));
+    if (grp > 0) {
+#pragma unroll
+      for (int q4 = 0; q4 < 2 * VH; ++q4)
+        lds_o[(grp * 2 * VH + q4) * tpg + t] =
+            f32x4_t{acc[4 * q4], acc[4 * q4 + 1], acc[4 * q4 + 2], acc[4 * q4 + 3]};
+      lds_ml[grp * tpg + t] = make_float2(M, Lsum);
+    }
+    __syncthreads();
+    if (grp > 0 || !row_ok) return;
+    for (int gi = 1; gi < c.groups; ++gi) {
+      const float2 ml = lds_ml[gi * tpg + t];
+      if (ml.x == -INFINITY) continue;
+      const float Mn = fmaxf(M, ml.x);
+      const float c_old = fast_exp2(M - Mn), c_new = fast_exp2(ml.x - Mn);
+#pragma unroll
+      for (int q4 = 0; q4 < 2 * VH; ++q4) {
+        const f32x4_t v = lds_o[(gi * 2 * VH + q4) * tpg + t];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[4 * q4 + e] = acc[4 * q4 + e] * c_old + v[e] * c_new;
+      }
+      Lsum = Lsum * c_old + ml.y * c_new;
       M = Mn;
     }
   }
@@ -838,11 +883,27 @@ static int decode_launch(const fw_decode_params *p, void *ws, size_t ws_bytes,
   c.lse = p->lse;
   c.v_descale = p->v_descale;
   c.vd = p->v_descale_ptr;
-  const dim3 grid(p->nheads_k * L.n_qtiles, p->batch);
-  const int threads = 16 * L.rows_item;  // rows_item <= 16
-  if (p->head_dim == 256) fw_decode_combine<256><<<grid, threads, 0, s>>>(c);
-  else if (p->head_dim == 64) fw_decode_combine<64><<<grid, threads, 0, s>>>(c);
-  else fw_decode_combine<128><<<grid, threads, 0, s>>>(c);
+  // A row has about nw / batch + 1 segments: groups of eight (one batch of
+  // loads each) as far as a block's threads allow, fewer rows per block then,
+  // and four waves a block at least (one long row among short ones has up to
+  // nw segments: 32,000 keys beside 63 rows of 60, 73 -> 53 us; four groups at
+  // 16 rows, 1,024 threads for rows of three segments, cost a batch of 128 fp8
+  // verify windows 1%).  One row of 4,001 keys, 32/8 heads, has 126 segments:
+  // one group merged them in 23 us of dependent loads, 16 groups in 6.
+  auto merge = [&](auto dc) {
+    constexpr int D = decltype(dc)::value;
+    c.groups = 1;
+    while (16 * L.rows_item * c.groups < 256) c.groups *= 2;
+    while (c.groups < 16 && c.groups * 8 * p->batch < L.nw) c.groups *= 2;
+    c.rows_blk = std::min(L.rows_item, std::max(1, kMergeThreads<D> / (16 * c.groups)));
+    const dim3 grid(p->nheads_k * L.n_qtiles * ceil_div(L.rows_item, c.rows_blk), p->batch);
+    const int threads = 16 * c.rows_blk * c.groups;
+    const size_t lds = c.groups > 1 ? (size_t)threads * (8 * kVH<D> + 2) * sizeof(float) : 0;
+    fw_decode_combine<D><<<grid, threads, lds, s>>>(c);
+  };
+  if (p->head_dim == 256) merge(std::integral_constant<int, 256>());
+  else if (p->head_dim == 64) merge(std::integral_constant<int, 64>());
+  else merge(std::integral_constant<int, 128>());
   return check_launch("fw_decode_combine");
 }
 

@@ -354,3 +354,29 @@ def test_decode_head_dims(dtype, seqlen_q, hd):
     ro, rl = oracle(case, q, exp_pool, causal=seqlen_q > 1)
     assert_close(out.float().cpu().numpy(), ro, fp8=dtype != "bf16")
     assert_lse(lse.cpu().numpy(), rl)
+
+
+@pytest.mark.parametrize("nheads,nheads_k,sq,d", [
+    (2, 2, 1, 128),   # 1 row a tile: 16 groups, one row per block
+    (6, 2, 1, 64),    # 3 rows
+    (8, 2, 4, 128),   # 16 rows: 4 per block at 16 groups
+    (10, 2, 5, 256),  # 25 rows in two q tiles: 2 per block at 16 groups
+])
+@pytest.mark.parametrize("lengths", [
+    (33,), (3000,),      # two segments for 16 groups; a segment per group and more
+    (2900, 0, 40, 7),    # one long row among short and empty ones
+])
+def test_merge_segment_groups(nheads, nheads_k, sq, d, lengths):
+    announce(f"decode merge h{nheads}/{nheads_k} sq{sq} d{d} lengths {lengths}")
+    rng = np.random.default_rng(31)
+    b = len(lengths)
+    case = PagedCase(rng, batch=b, nheads=nheads, nheads_k=nheads_k, lengths=lengths,
+                     new_tokens=[sq] * b, head_dim=d)
+    q = randn(rng, (b, sq, nheads, d))
+    sinks = rng.standard_normal(nheads).astype(np.float32) if sq == 1 else None
+    out, lse, pool = run_decode(case, q, causal=True, sinks=sinks)
+    exp_pool = case.expected_pool()
+    np.testing.assert_array_equal(codes_of(pool), exp_pool)
+    ro, rl = oracle(case, q, exp_pool, causal=True, sinks=sinks)
+    assert_close(out.float().cpu().numpy(), ro)
+    assert_lse(lse.cpu().numpy(), rl)
