@@ -15,8 +15,10 @@
 //   fw_prefill_pp_pair_kernel, fw_prefill_d256_pair_kernel
 //                              the same on large dense grids, two mirrored q
 //                              tiles per workgroup
-//   fw_prefill_d64_kernel      head dims 64/64, bf16 K/V: 4 waves, three
-//                              workgroups per CU
+//   fw_prefill_fr_kernel       head dims 64/64 and 192/128 (bf16 K/V), and
+//                              small dense grids at 64, 128 and 192/128:
+//                              free-running waves, the key tiles of a q tile
+//                              split over waves where the grid is small
 //   fw_prefill_staged_kernel   the other head dims (96, 192, 384, 512, mixed
 //                              q / v widths) and fp8 pools at 64: K/V staged
 //                              in registers
@@ -1822,43 +1824,87 @@ __global__ __launch_bounds__(256, 1) void fw_prefill_d256_pair_kernel(PrefillArg
 }
 
 // ---------------------------------------------------------------------------
-// head_dim 64, bf16 K/V: workgroup = 4 waves of 32 q rows each (2^hpw_shift
-// <= 4 query heads of a GQA group over the same rows), three workgroups per
-// CU.  A 64-key tile is 16 MFMAs (512 cycles) and about as much VALU work (32
-// exponentials, 32 adds, 16 packs) a wave, so neither pipe can hide behind
-// the other inside one wave, and a single wave issues VALU at half the SIMD's
-// rate; three free-running waves per SIMD (up to 168 registers each) overlap
-// the two.  K/V tiles (8 KiB each, 128-byte rows) rotate through three LDS
-// buffers, copied straight from global memory two tiles ahead; one barrier per
-// tile.  Measured, 4 x 32/8 heads x 1999 tokens, causal: 79.8 us, 820 TFLOP/s
+// bf16 K/V, free-running waves: workgroup = KG key groups x RW waves of 32 q
+// rows (2^hpw_shift <= RW query heads of a GQA group over the same rows).  A
+// group walks every KG-th 64-key tile; its RW waves share a tile through LDS,
+// copied straight from global memory.  Three forms:
+//   KG = 1, RW = 4: several workgroups per CU.  Where a tile's matrix work is
+//     no longer than its softmax (head dim 64: 16 MFMAs, 512 cycles, beside 32
+//     exponentials, 32 adds and 16 packs a wave), neither pipe can hide behind
+//     the other inside one wave and a single wave issues VALU at half the
+//     SIMD's rate; two or three waves per SIMD that are not in step overlap
+//     the two.
+//   KG = 2, RW = 4: grids that leave CUs idle; 8 waves on 128 rows.
+//   RW = 1: the smallest grids; every wave has LDS of its own and no barrier
+//     runs in the loop, so 32 rows of one head finish after 1 / KG of their
+//     key tiles.
+// The groups' (m, l, O) are merged through LDS in group order at the end.
+// Measured, causal: 64/64, 4 x 32/8 heads x 1999 tokens 79.8 us, 820 TFLOP/s
 // (the register-staged kernel at two waves per SIMD: 137.7 us, 476); with
 // softcap 50 91.8 (151.6) us; 8K and 16K tokens 962 and 1,025 TFLOP/s, at which
-// the chip's power sets the clock (1.96 GHz).  Four waves per SIMD spill (128
-// registers): 120 us.  Without the exponentials 66 us, without the copies 69.
-constexpr int kD6Waves = 4;
-constexpr int kD6RowB = 128;                // LDS bytes of one key row
-constexpr int kD6TileB = kKT * kD6RowB;     // 8 KiB per K or V tile
-constexpr int kD6Buf = 2 * kD6TileB;        // [K tile | V tile]
-// 16-byte chunk swizzle of a 128-byte LDS row: two rows fill the 64 banks, so
-// 16 consecutive rows need 8 distinct values over r / 2 (plain 16-byte reads),
-// and rows r and r + 2 of an aligned key quad must differ in bit 2 (the four
-// rows x four chunks that 32 lanes of a transposing read cover).
-__device__ __forceinline__ int swz64(int r) {
-  return 4 * ((r >> 1) & 1) + 2 * ((r >> 2) & 1) + ((r >> 3) & 1);
+// the chip's power sets the clock (1.96 GHz); four waves per SIMD spill (128
+// registers): 120 us; without the exponentials 66 us, without the copies 69.
+// 192/128, 64/8 heads x 4096 tokens 288 us, 16/16 x 2048 x 3000 62 us and 52 us
+// in the mid form (register-staged: 129).  What the forms are worth on smaller
+// grids stands at dense_form.
+constexpr int kFrKeys = 64;
+// 16-byte chunk swizzle of LDS row r: 256-byte rows as in the ping-pong kernel
+// (swz).  Rows of 128 and 384 bytes alternate between the halves of the 64
+// banks, so 16 consecutive rows need 8 distinct values over r / 2 (plain
+// 16-byte reads), and rows r and r + 2 of an aligned key quad must differ in
+// bit 2 (the four rows x four chunks that 32 lanes of a transposing read cover).
+template <int ROWB>
+__device__ __forceinline__ int row_swizzle(int r) {
+  if constexpr (ROWB == 256) return swz(r);
+  else return 4 * ((r >> 1) & 1) + 2 * ((r >> 2) & 1) + ((r >> 3) & 1);
 }
 
-template <int MODE, bool SOFTCAP>
-__global__ __launch_bounds__(256, 3) void fw_prefill_d64_kernel(PrefillArgs a) {
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[3 * kD6Buf];
+// Copies 16 rows of ROWB bytes (row stride st bytes from base; rows past lim
+// re-read row lim) to LDS at dst, swizzled: instruction i writes 1 KiB, lane l
+// the physical chunk of byte 1024 i + 16 l.
+template <int ROWB>
+__device__ __forceinline__ void copy_rows16(const uint8_t *base, uint32_t st, uint32_t lim,
+                                            uint32_t dst, int lane) {
+  auto voff = [&](int i) __attribute__((always_inline)) {
+    uint32_t row, ch;
+    if constexpr (ROWB == 384) {  // three instructions cover eight rows
+      const uint32_t o = 64u * (i % 3) + lane;
+      row = 8u * (i / 3) + o / 24u;
+      ch = o % 24u;
+    } else {
+      constexpr int LPR = ROWB / 16;
+      row = (64 / LPR) * i + lane / LPR;
+      ch = lane % LPR;
+    }
+    return __umul24(min(row, lim), st) + 16u * (ch ^ (uint32_t)row_swizzle<ROWB>(row));
+  };
+#pragma unroll
+  for (int i = 0; i < 16 * ROWB / 1024; i += 2)
+    lds_dma16x2(base, voff(i), voff(i + 1), dst + 1024u * i);
+}
+
+template <int MODE, bool SOFTCAP, int D, int DV, int RW, int KG, int BUFS, int OCC>
+__global__ __launch_bounds__(64 * RW * KG, OCC) void fw_prefill_fr_kernel(PrefillArgs a) {
+  static_assert(BUFS > 1 || RW == 1, "one buffer: private to a wave");
+  constexpr int kKB = 2 * D, kVB = 2 * DV;                  // row bytes
+  constexpr int kKTile = kFrKeys * kKB, kBuf = kKTile + kFrKeys * kVB;
+  constexpr int kRows = kFrKeys / RW;                       // key rows a wave copies
+  constexpr int kNK = kRows * kKB / 1024, kNV = kRows * kVB / 1024;  // its copies per tile
+  constexpr int NJ = D / 16, NC = DV / 32;
+  constexpr int kMergeB = (KG - 1) * RW * 32 * DV * 4;      // O of groups 1 .., then (m, l)
+  constexpr int kLdsEnd = kMergeB + (KG - 1) * RW * 32 * 8;
+  constexpr int kLds = KG * BUFS * kBuf > kLdsEnd ? KG * BUFS * kBuf : kLdsEnd;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLds];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = wave % RW, kg = wave / RW;
   const int n = lane & 31;
   const int g = lane >> 5;
-  // wave w: head hg * 2^hpw_shift + (w >> wph_shift), rows q0 + 32 rb ..
-  const int wph_shift = 2 - a.hpw_shift;
+  // wave w of a group: head hg * 2^hpw_shift + (w >> wph_shift), rows q0 + 32 rb ..
+  const int wph_shift = (RW == 4 ? 2 : 0) - a.hpw_shift;
   const int rb = w & ((1 << wph_shift) - 1);
-  const int R = (32 * kD6Waves) >> a.hpw_shift;
+  const int R = (32 * RW) >> a.hpw_shift;
 
   // ------------------------------------------------------------ tile decode
   int b = 0, hg, seq = 0, q0, sq_len, sk_len, qtok0 = 0, kbase = 0;
@@ -1880,9 +1926,10 @@ __global__ __launch_bounds__(256, 3) void fw_prefill_d64_kernel(PrefillArgs a) {
     if (seq < 0) {  // packed padding rows: out 0, lse -inf
       const int hp = (hg << a.hpw_shift) + (w >> wph_shift);
       const int r0 = q0 + 32 * rb + n;
-      if (r0 < a.Sq) {
+      if (r0 < a.Sq && kg == 0) {
         uint16_t *o = a.out + (size_t)hp * a.osh + (size_t)r0 * a.ost;
-        for (int d = g * 32; d < g * 32 + 32; d += 8) *(u32x4_t *)(o + d) = u32x4_t{0, 0, 0, 0};
+        for (int d = g * (DV / 2); d < (g + 1) * (DV / 2); d += 8)
+          *(u32x4_t *)(o + d) = u32x4_t{0, 0, 0, 0};
         if (a.lse && g == 0) a.lse[(size_t)hp * a.lsh + r0] = -INFINITY;
       }
       return;
@@ -1918,79 +1965,94 @@ __global__ __launch_bounds__(256, 3) void fw_prefill_d64_kernel(PrefillArgs a) {
   const int qrow = q0 + 32 * rb + n;
   const bool row_ok = qrow < sq_len;
   const int r_lo = row_lo(qrow), r_hi = row_hi(qrow);
-  const int t_begin = wg_hi > wg_lo ? wg_lo / kKT : 0;
-  const int t_end = wg_hi > wg_lo ? (wg_hi + kKT - 1) / kKT : 0;
-  const int T = t_end - t_begin;
+  const int t_begin = wg_hi > wg_lo ? wg_lo / kFrKeys : 0;
+  const int t_end = wg_hi > wg_lo ? (wg_hi + kFrKeys - 1) / kFrKeys : 0;
+  // steps of the workgroup, and this group's tiles (t_begin + KG t + kg)
+  const int steps = (t_end - t_begin + KG - 1) / KG;
+  const int T = (t_end - t_begin - kg + KG - 1) / KG;
 
-  // ---- copies: tile j lands in buffer j % 3; this wave moves key rows 16w ..
-  // 16w + 15 of K and of V, eight rows per instruction: lane l writes
-  // physical chunk l % 8 of row 8i + l / 8, which holds logical chunk
-  // (l % 8) ^ swz64(row).  The 16 rows lie on one page (P % 16 == 0).
+  // ---- copies: tile t of the group lands in its buffer t % BUFS; this wave
+  // moves key rows kRows w .. of K and of V, 16 at a time (16 rows lie on one
+  // page: P % 16 == 0)
   const uint32_t lds0 = (uint32_t)(uintptr_t)(FW_LDS uint8_t *)lds;
+  const uint32_t ldsg = lds0 + (uint32_t)(BUFS == 1 ? wave : kg * BUFS) * kBuf;
   uint32_t kstB, vstB;
   const uint8_t *kbase_p = nullptr, *vbase_p = nullptr;
   if constexpr (MODE == FW_KV_PAGED) {
-    kstB = vstB = (uint32_t)a.CH * kD6RowB;
+    kstB = vstB = (uint32_t)a.CH * kKB;
   } else {
     kstB = 2u * (uint32_t)a.kst;
     vstB = 2u * (uint32_t)a.vst;
     kbase_p = a.k + 2 * ((size_t)b * a.ksb + (size_t)hk * a.ksh + (size_t)kbase * a.kst);
     vbase_p = a.v + 2 * ((size_t)b * a.vsb + (size_t)hk * a.vsh + (size_t)kbase * a.vst);
   }
-  const uint32_t lr = lane >> 3;
-  const uint32_t lch = 16u * (uint32_t)((lane & 7) ^ (4 * ((lane >> 4) & 1) + 2 * ((lane >> 5) & 1)));
-  auto dma = [&](int j, int buf) __attribute__((always_inline)) {
+  constexpr int kCopyK = 1, kCopyV = 2;
+  auto dma = [&](int t, int buf, int what) __attribute__((always_inline)) {
     const int kmax = sk_len - 1;
-    int key0 = min((t_begin + j) * kKT + 16 * w, kmax);
-    const uint8_t *kp, *vp;
-    bool bad = false;
-    if constexpr (MODE == FW_KV_PAGED) {
-      key0 &= ~15;
-      const int page = a.table[(size_t)seq * a.max_pages + key0 / a.P];
-      bad = page < 0 || page >= a.num_pages;  // never dereferenced: reads the zero rows
-      kp = a.k + (((size_t)page * a.P + key0 % a.P) * a.CH + 2 * hk) * kD6RowB;
-      if (bad) kp = kZeroKV;
-      vp = kp + kD6RowB;
-    } else {
-      kp = kbase_p + (size_t)key0 * kstB;
-      vp = vbase_p + (size_t)key0 * vstB;
+#pragma unroll
+    for (int rg = 0; rg < kRows / 16; ++rg) {
+      const int row0 = kRows * w + 16 * rg;
+      int key0 = min((t_begin + KG * t + kg) * kFrKeys + row0, kmax);
+      const uint8_t *kp, *vp;
+      bool bad = false;
+      if constexpr (MODE == FW_KV_PAGED) {
+        key0 &= ~15;
+        const int page = a.table[(size_t)seq * a.max_pages + key0 / a.P];
+        bad = page < 0 || page >= a.num_pages;  // never dereferenced: reads the zero rows
+        kp = a.k + (((size_t)page * a.P + key0 % a.P) * a.CH + 2 * hk) * kKB;
+        if (bad) kp = kZeroKV;
+        vp = kp + kKB;
+      } else {
+        kp = kbase_p + (size_t)key0 * kstB;
+        vp = vbase_p + (size_t)key0 * vstB;
+      }
+      const uint32_t lim = bad ? 0u : (uint32_t)(kmax - key0);
+      const uint32_t d = ldsg + (uint32_t)buf * kBuf;
+      if (what & kCopyK) copy_rows16<kKB>(kp, kstB, lim, d + row0 * kKB, lane);
+      if (what & kCopyV) copy_rows16<kVB>(vp, vstB, lim, d + kKTile + row0 * kVB, lane);
     }
-    const uint32_t lim = bad ? 0u : (uint32_t)(kmax - key0);
-    const uint32_t ra = min(lr, lim), rc = min(lr + 8u, lim);  // rows past the last key re-read it
-    const uint32_t d = lds0 + (uint32_t)(16 * w * kD6RowB) + (uint32_t)buf * kD6Buf;
-    lds_dma16x2(kp, __umul24(ra, kstB) + lch, __umul24(rc, kstB) + (lch ^ 16u), d);
-    lds_dma16x2(vp, __umul24(ra, vstB) + lch, __umul24(rc, vstB) + (lch ^ 16u), d + kD6TileB);
   };
-  if (T > 0) dma(0, 0);
-  if (T > 1) dma(1, 1);
+  if constexpr (BUFS == 1) {
+    if (T > 0) {
+      dma(0, 0, kCopyK);
+      dma(0, 0, kCopyV);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < BUFS - 1; ++i)
+      if (i < T) dma(i, i, kCopyK | kCopyV);
+  }
 
   // ------------------------------------------------------------ Q^T operand
-  bf16x8_t qop[4];
+  bf16x8_t qop[NJ];
   {
     const uint16_t *qp = a.q + (size_t)b * a.qsb + (size_t)h * a.qsh +
                          (size_t)(qtok0 + (row_ok ? qrow : 0)) * a.qst;
     const float qs = row_ok ? q_scale_of(a) : 0.f;  // rows past the end get q = 0
-    load_q_operand<64>(a, qp, g, qs, qrow + off, qop);
+    load_q_operand<D>(a, qp, g, qs, qrow + off, qop);
   }
   // ---- LDS operand addressing (per-lane byte offsets within a buffer):
-  // K row 32st + n, chunk 2j + g; V rows 16u + 8r + 4g + tr_a, dims 32c +
-  // 16(G & 1) + 4 tr_b (transposing reads, as in the head_dim-128 kernel).
-  uint32_t kofs[4], vofs[2][2];
+  // K row 32st + n, chunk 2j + g, where steps j and j + KJ are 2 KJ chunks
+  // apart; V rows 16u + 8r + 4g + tr_a, dims 32c + 16(G & 1) + 4 tr_b
+  // (transposing reads, as in the ping-pong kernel)
+  constexpr int KJ = kKB == 256 ? 8 : 4;
+  constexpr int VC = kVB == 256 ? 4 : 2;
+  uint32_t kofs[KJ], vofs[VC][2];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) kofs[j] = lds0 + n * kD6RowB + 16 * ((2 * j + g) ^ swz64(n));
+  for (int j = 0; j < KJ; ++j) kofs[j] = ldsg + n * kKB + 16 * ((2 * j + g) ^ row_swizzle<kKB>(n));
   const int tr_a = (lane >> 2) & 3, tr_b = lane & 3;
 #pragma unroll
-  for (int c = 0; c < 2; ++c)
+  for (int c = 0; c < VC; ++c)
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
       const int row = 8 * r + 4 * g + tr_a;
       const int chunk = 4 * c + 2 * ((lane >> 4) & 1) + (tr_b >> 1);
-      vofs[c][r] = lds0 + kD6TileB + row * kD6RowB + 16 * (chunk ^ swz64(row)) + 8 * (tr_b & 1);
+      vofs[c][r] = ldsg + kKTile + row * kVB + 16 * (chunk ^ row_swizzle<kVB>(row)) + 8 * (tr_b & 1);
     }
 
-  f32x16_t oacc[2];
+  f32x16_t oacc[NC];
 #pragma unroll
-  for (int c = 0; c < 2; ++c)
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int e = 0; e < 16; ++e) oacc[c][e] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
@@ -2001,30 +2063,58 @@ __global__ __launch_bounds__(256, 3) void fw_prefill_d64_kernel(PrefillArgs a) {
   for (int e = 0; e < 16; ++e) neg_m[e] = 0.f;
 
   auto step = [&](const int t, const auto bi) __attribute__((always_inline)) {
-    constexpr uint32_t buf = decltype(bi)::value * kD6Buf;
-    // this wave's copies of tile t are complete (tile t + 1's four may be in
-    // flight); the barrier publishes every wave's and frees tile t - 1's buffer
-    if (t + 1 < T) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (t + 2 < T) dma(t + 2, (decltype(bi)::value + 2) % 3);
-    const int kb = (t_begin + t) * kKT;
-    if (kb >= w_hi || kb + kKT <= w_lo) return;  // this wave's rows see nothing here
+    constexpr int B = decltype(bi)::value;
+    constexpr uint32_t buf = B * kBuf;
+    if constexpr (BUFS > 1) {
+      // this wave's copies of tile t are complete (with three buffers tile t +
+      // 1's may be in flight); the barrier publishes every wave's and frees
+      // tile t - 1's buffer
+      if (BUFS == 3 && t + 1 < T) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kNK + kNV) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (t + BUFS - 1 < T) dma(t + BUFS - 1, (B + BUFS - 1) % BUFS, kCopyK | kCopyV);
+    } else {
+      // K of tile t is in; V's copies (issued after it) may be in flight
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kNV) : "memory");
+    }
+    const int kb = (t_begin + KG * t + kg) * kFrKeys;
+    // no tile left, or this wave's rows see nothing of it
+    if (BUFS > 1 && (t >= T || kb >= w_hi || kb + kFrKeys <= w_lo)) return;
     f32x16_t sacc[2];
+    {
+      // K operands run KP steps ahead of their MFMAs, pinned by fences where
+      // few waves hide the reads (at head dim 64, three waves per SIMD, the
+      // compiler's own order measured the same)
+      constexpr bool kPin = D > 64;
+      constexpr int NS = 2 * NJ, KP = 4;
+      bf16x8_t kop[KP];
+      auto kread = [&](int i) __attribute__((always_inline)) {
+        const int j = i >> 1, st = i & 1;
+        kop[i % KP] = __builtin_bit_cast(
+            bf16x8_t, *(const FW_LDS u32x4_t *)(kofs[j % KJ] + buf + 32u * KJ * (j / KJ) + 32u * kKB * st));
+      };
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+      for (int i = 0; i < KP; ++i) kread(i);
+      if constexpr (kPin) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        const bf16x8_t ko = __builtin_bit_cast(
-            bf16x8_t, *(const FW_LDS u32x4_t *)(kofs[j] + buf + 32 * kD6RowB * st));
+      for (int i = 0; i < NS; ++i) {
+        const int j = i >> 1, st = i & 1;
+        const bf16x8_t ko = kop[i % KP];
+        if (i + KP < NS) kread(i + KP);
         if (SOFTCAP && j == 0) sacc[st] = mfma32(ko, qop[j], f32x16_t{});
         else sacc[st] = mfma32(ko, qop[j], j == 0 ? neg_m : sacc[st]);
+        if constexpr (kPin) __builtin_amdgcn_sched_barrier(0);
       }
+    }
+    if constexpr (BUFS == 1) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the K rows are read
+      if (t + 1 < T) dma(t + 1, 0, kCopyK);
+    }
     // online softmax against the static anchor, as in the ping-pong kernel
     const float m_qk = m_run == -INFINITY ? 0.f : m_run;
     if constexpr (SOFTCAP) softcap_scores<2, 16, true>(sacc, a.softcap_log2, m_qk);
-    const bool full = kb >= row_lo(w_last) && kb + kKT <= row_hi(w_first) && kb + kKT <= sk_len;
+    const bool full = kb >= row_lo(w_last) && kb + kFrKeys <= row_hi(w_first) && kb + kFrKeys <= sk_len;
     bool row_has_key = true;
     if (!full) {
 #pragma unroll
@@ -2034,7 +2124,7 @@ __global__ __launch_bounds__(256, 3) void fw_prefill_d64_kernel(PrefillArgs a) {
           const int key = kb + 32 * st + 8 * (e >> 2) + 4 * g + (e & 3);
           sacc[st][e] = (key >= r_lo && key < r_hi) ? sacc[st][e] : -INFINITY;
         }
-      row_has_key = max(r_lo, kb) < min(r_hi, kb + kKT);
+      row_has_key = max(r_lo, kb) < min(r_hi, kb + kFrKeys);
     }
     bf16x8_t pop[4];
     float psum;
@@ -2069,34 +2159,99 @@ __global__ __launch_bounds__(256, 3) void fw_prefill_d64_kernel(PrefillArgs a) {
       exponentiate(m_use - m_qk);
       l_run *= alpha;
 #pragma unroll
-      for (int c = 0; c < 2; ++c) oacc[c] *= alpha;
+      for (int c = 0; c < NC; ++c) oacc[c] *= alpha;
       if constexpr (!SOFTCAP) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) neg_m[e] = -m_use;
       }
     }
     l_run += psum;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
+    if constexpr (BUFS == 1) {  // V of tile t is in; K of tile t + 1 may be in flight
+      if (t + 1 < T) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kNK) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    {
+      constexpr bool kPin = D > 64;
+      constexpr int NS = 4 * NC, VP = 3;
+      bf16x8_t vop[VP];
+      auto vread = [&](int i) __attribute__((always_inline)) {
+        const int u = i / NC, c = i % NC;
         const v4i16_t p0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (FW_LDS v4i16_t *)(vofs[c][0] + buf + 16 * u * kD6RowB));
+            (FW_LDS v4i16_t *)(vofs[c][0] + buf + 16 * u * kVB));
         const v4i16_t p1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (FW_LDS v4i16_t *)(vofs[c][1] + buf + 16 * u * kD6RowB));
-        const bf16x8_t vo = __builtin_bit_cast(
+            (FW_LDS v4i16_t *)(vofs[c][1] + buf + 16 * u * kVB));
+        vop[i % VP] = __builtin_bit_cast(
             bf16x8_t, __builtin_shufflevector(p0, p1, 0, 1, 2, 3, 4, 5, 6, 7));
-        oacc[c] = mfma32(vo, pop[u], oacc[c]);
+      };
+#pragma unroll
+      for (int i = 0; i < VP; ++i) vread(i);
+      if constexpr (kPin) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < NS; ++i) {
+        const bf16x8_t vo = vop[i % VP];
+        if (i + VP < NS) vread(i + VP);
+        oacc[i % NC] = mfma32(vo, pop[i / NC], oacc[i % NC]);
+        if constexpr (kPin) __builtin_amdgcn_sched_barrier(0);
       }
+    }
+    if constexpr (BUFS == 1) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the V rows are read
+      if (t + 1 < T) dma(t + 1, 0, kCopyV);
+    }
   };
-  for (int t = 0; t < T; t += 3) {
-    step(t, std::integral_constant<int, 0>());
-    if (t + 1 < T) step(t + 1, std::integral_constant<int, 1>());
-    if (t + 2 < T) step(t + 2, std::integral_constant<int, 2>());
+  static_assert(VC == NC, "one V address pair per 32-dim block");
+  if constexpr (BUFS == 1) {
+    for (int t = 0; t < T; ++t) step(t, std::integral_constant<int, 0>());
+  } else {
+    for (int t = 0; t < steps; t += BUFS) {
+      step(t, std::integral_constant<int, 0>());
+      if (t + 1 < steps) step(t + 1, std::integral_constant<int, 1>());
+      if constexpr (BUFS == 3) {
+        if (t + 2 < steps) step(t + 2, std::integral_constant<int, 2>());
+      }
+    }
   }
 
   // ------------------------------------------------------------ epilogue
   l_run += __shfl_xor(l_run, 32, 64);
+  __syncthreads();  // every wave's LDS reads of the loop are done
+  if constexpr (KG > 1) {
+    // groups 1 .. hand their (m, l, O) to group 0 through LDS: each wave's
+    // registers as 16-byte pieces at lane order
+    const uint32_t ml0 = lds0 + kMergeB + 8u * (w * 32 + n);  // 256 RW bytes per group
+    constexpr int kWaveB = 32 * DV * 4;
+    if (kg > 0) {
+      const uint32_t o = lds0 + (uint32_t)((kg - 1) * RW + w) * kWaveB + 16u * lane;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr)
+          *(FW_LDS f32x4_t *)(o + 1024u * (4 * c + rr)) =
+              f32x4_t{oacc[c][4 * rr], oacc[c][4 * rr + 1], oacc[c][4 * rr + 2], oacc[c][4 * rr + 3]};
+      if (g == 0) *(FW_LDS f32x2_t *)(ml0 + 256u * RW * (kg - 1)) = f32x2_t{m_run, l_run};
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll 1
+    for (int k = 0; k < KG - 1; ++k) {
+      const f32x2_t x = *(const FW_LDS f32x2_t *)(ml0 + 256u * RW * k);
+      const float Mx = fmaxf(m_run, x.x);
+      const float f0 = m_run == -INFINITY ? 0.f : fast_exp2(m_run - Mx);
+      const float f1 = x.x == -INFINITY ? 0.f : fast_exp2(x.x - Mx);
+      const uint32_t o = lds0 + (uint32_t)(k * RW + w) * kWaveB + 16u * lane;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+          const f32x4_t v = *(const FW_LDS f32x4_t *)(o + 1024u * (4 * c + rr));
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            oacc[c][4 * rr + e] = fmaf(v[e], f1, oacc[c][4 * rr + e] * f0);
+        }
+      l_run = fmaf(x.y, f1, l_run * f0);
+      m_run = Mx;
+    }
+  }
   float M = m_run, Lsum = l_run, oscale = 1.f;
   if (a.sinks) {
     const float sk = a.sinks[h] * kLog2e;
@@ -2110,22 +2265,23 @@ __global__ __launch_bounds__(256, 3) void fw_prefill_d64_kernel(PrefillArgs a) {
   }
   const bool any = Lsum > 0.f && l_run > 0.f;
   const float scale = any ? oscale * v_descale_of(a) / Lsum : 0.f;
-  // O goes out as whole 128-byte rows, staged through the wave's 4 KiB of LDS
-  __syncthreads();  // every wave's LDS reads of the loop are done
+  // O goes out as whole rows, staged through LDS: the wave's own merge slot
+  // (or, with one group, its share of the buffers), which no other wave reads
   {
-    const uint32_t wbase = lds0 + (uint32_t)w * 4096u;
+    const uint32_t wbase = lds0 + (uint32_t)w * (32u * DV * 4);
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
         const u32x2_t wv = {pack_bf16(oacc[c][4 * rr] * scale, oacc[c][4 * rr + 1] * scale),
                             pack_bf16(oacc[c][4 * rr + 2] * scale, oacc[c][4 * rr + 3] * scale)};
-        *(FW_LDS u32x2_t *)(wbase + n * kD6RowB + 16 * ((4 * c + rr) ^ swz64(n)) + 8 * g) = wv;
+        *(FW_LDS u32x2_t *)(wbase + n * kVB + 16 * ((4 * c + rr) ^ row_swizzle<kVB>(n)) + 8 * g) = wv;
       }
+    constexpr int LPR = kVB / 16;  // lanes per row
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 8 * i + (lane >> 3), cc = lane & 7;
-      const u32x4_t v = *(const FW_LDS u32x4_t *)(wbase + r * kD6RowB + 16 * (cc ^ swz64(r)));
+    for (int i = 0; i < 32 * LPR / 64; ++i) {
+      const int r = (64 / LPR) * i + lane / LPR, cc = lane % LPR;
+      const u32x4_t v = *(const FW_LDS u32x4_t *)(wbase + r * kVB + 16 * (cc ^ row_swizzle<kVB>(r)));
       const int grow = q0 + 32 * rb + r;
       if (grow < sq_len)
         __builtin_nontemporal_store(v, (u32x4_t *)(a.out + (size_t)b * a.osb + (size_t)h * a.osh +
@@ -2306,15 +2462,22 @@ static bool use_pingpong(const fw_prefill_params *p) {
          head_dim_v_of(p) == 128;
 }
 
-static bool use_d64(const fw_prefill_params *p) {
-  return p->kv_dtype == FW_BF16 && p->head_dim == 64 && head_dim_v_of(p) == 64;
+static bool use_fr(const fw_prefill_params *p) {
+  return p->kv_dtype == FW_BF16 && ((p->head_dim == 64 && head_dim_v_of(p) == 64) ||
+                                    (p->head_dim == 192 && head_dim_v_of(p) == 128));
 }
 
+// Forms of a dense call at head dims 64/64, 128/128 and 192/128 by the size of
+// its grid: kFormLarge is the kernel the head dim runs everywhere, the others
+// fw_prefill_fr_kernel with the key tiles of a q tile split over waves.
+constexpr int kFormLarge = 0, kFormMid = 1, kFormSmall = 2;
+
 // log2 of the query heads per workgroup: the largest power of two that
-// divides the GQA group size (1 for MHA), up to the workgroup's waves (8 in
-// the ping-pong kernel, 4 in the head_dim-64 one); the other kernels take one.
-static int pp_head_shift(const fw_prefill_params *p) {
-  const int most = use_pingpong(p) ? 3 : use_d64(p) ? 2 : 0;
+// divides the GQA group size (1 for MHA), up to the workgroup's waves that
+// hold different rows (8 in the ping-pong kernel, 4 in fw_prefill_fr_kernel, 1
+// in its small form); the other kernels take one.
+static int pp_head_shift(const fw_prefill_params *p, int form = kFormLarge) {
+  const int most = form == kFormMid ? 2 : form == kFormSmall ? 0 : use_pingpong(p) ? 3 : use_fr(p) ? 2 : 0;
   const int G = p->nheads_k > 0 ? p->nheads / p->nheads_k : 1;
   int sh = 0;
   while (sh < most && G % (2 << sh) == 0) ++sh;
@@ -2322,8 +2485,48 @@ static int pp_head_shift(const fw_prefill_params *p) {
 }
 
 // q rows per schedule slot (and per dense q tile).
-static int prefill_tile_rows(const fw_prefill_params *p) {
-  return (use_pingpong(p) ? kPPRows : kQT) >> pp_head_shift(p);
+static int prefill_tile_rows(const fw_prefill_params *p, int form = kFormLarge) {
+  if (form == kFormSmall) return 32;
+  return (form == kFormLarge && use_pingpong(p) ? kPPRows : kQT) >> pp_head_shift(p, form);
+}
+
+// The form of a dense call, by the workgroups each would launch on the CUs and
+// the key tiles T a q tile visits.  Measured (us per call, large / mid / small,
+// 256 CUs; heads x queries x keys):
+//   small, while one workgroup per 32 rows fits the CUs and T >= 8:
+//     128/128   8/2 x 512 x 512 17.8 / 13.2 / 11.3, 8/2 x 64 x 4096 76 / 49 / 31,
+//               8/2 x 1024 x 1024 26 / 18.6 / 15.1 (256 workgroups);
+//               T = 5 14.6 / 11.5 / 11.1, T = 2 11.4 / 8.9 / 9.3;
+//               two rounds of workgroups 16/4 x 1024 x 1024 26 / 19 / 23
+//     64/64     8/2 x 512 x 512 10.3 / 9.8 / 8.5, 8/2 x 64 x 4096 50 / 37 / 17
+//     192/128   8/2 x 512 x 512 15.5 / 15.2 / 12.4, 8/2 x 64 x 4096 78 / 58 / 35
+//   mid, while its 128-row workgroups fit the CUs (the other two from T = 8,
+//   where large runs several workgroups per CU):
+//     128/128   16/16 x 2048 x 2048 44.8 / 29.8, 16 x (16/16 x 256 x 256) 15.8 / 11.3
+//     64/64     16/16 x 2048 x 2048 28.4 / 21.9, T = 4 8.4 / 8.3
+//     192/128   16/16 x 2048 x 3000 62.1 / 51.9, T = 8 15.6 / 15.5, T = 4 11.3 / 12.1
+//   and up to two workgroups per CU when the causal mask makes long q tiles
+//   uneven (the second half of the workgroups evens them out):
+//     128/128   32/32 x 2048 x 2048 49.2 / 41.0 (not causal 58 / 66; 40 heads
+//               56 / 61), 32/8 x 1024 x 1024 twice 28.1 / 27.8
+//     64/64     32/32 x 2048 x 2048 29.3 / 26.6, 192/128 52.3 / 49.9
+static int dense_form(const fw_prefill_params *p) {
+  if (p->kv_mode != FW_KV_DENSE || !(use_fr(p) || use_pingpong(p))) return kFormLarge;
+  const long cus = device_cus();
+  auto grid = [&](int form) {
+    const int rows = prefill_tile_rows(p, form);
+    return (long)p->batch * (p->nheads >> pp_head_shift(p, form)) * ((p->seqlen_q + rows - 1) / rows);
+  };
+  const int right = p->causal ? 0 : p->window_right;
+  long keys = p->seqlen_k;
+  if (p->window_left >= 0 && right >= 0) keys = std::min(keys, (long)p->window_left + right + 32);
+  const long tiles = (keys + kFrKeys - 1) / kFrKeys;
+  if (grid(kFormSmall) <= cus && tiles >= 8) return kFormSmall;
+  const long mid = grid(kFormMid);
+  if (mid <= cus && (tiles >= 8 || use_pingpong(p))) return kFormMid;
+  const bool uneven = p->causal && p->window_left < 0 && 2l * p->seqlen_q >= p->seqlen_k;
+  if (mid <= 2 * cus && uneven && tiles >= 32) return kFormMid;
+  return kFormLarge;
 }
 
 }  // namespace fw
@@ -2363,8 +2566,9 @@ extern "C" size_t fw_prefill_workspace_bytes(const fw_prefill_params *p) {
 
 // Kernel choice (the host has checked the head dims): 128/128 -> the ping-pong
 // kernel, 256/256 -> the d256 kernel (fp8 pools widened as they land in LDS in
-// both), 64/64 with bf16 K/V -> the d64 kernel, everything else (head dims 96,
-// 192, 384, 512, head_dim_v != head_dim, fp8 pools at 64) -> the
+// both), 64/64 and 192/128 with bf16 K/V -> fw_prefill_fr_kernel (and small
+// dense grids at 128/128: dense_form), everything else (head dims 96, 192/192,
+// 384, 512, the other head_dim_v != head_dim, fp8 pools at 64) -> the
 // register-staged kernel.  A head_dim_v above 256 runs as
 // launches over chunks of v and out, which keeps O within one wave's
 // registers: 256 dims each at head dim 64, 128 each at head dims 384 and 512
@@ -2383,10 +2587,32 @@ template <int MODE, int KV, int D, int DV>
 static void launch_staged(const PrefillArgs &a, dim3 grid, hipStream_t s) {
   fw_prefill_staged_kernel<MODE, KV, D, DV><<<grid, 256, 0, s>>>(a);
 }
+template <int MODE, int D, int DV, int RW, int KG, int BUFS, int OCC>
+static void launch_fr(const PrefillArgs &a, dim3 grid, hipStream_t s) {
+  constexpr int threads = 64 * RW * KG;
+  if (a.softcap_log2 != 0.f)
+    fw_prefill_fr_kernel<MODE, true, D, DV, RW, KG, BUFS, OCC><<<grid, threads, 0, s>>>(a);
+  else
+    fw_prefill_fr_kernel<MODE, false, D, DV, RW, KG, BUFS, OCC><<<grid, threads, 0, s>>>(a);
+}
 template <int MODE>
 static void launch_mode(const PrefillArgs &a, dim3 grid, int kv_dtype, int d, int dv,
-                        hipStream_t s) {
+                        hipStream_t s, int form = kFormLarge) {
   if (kv_dtype == FW_BF16) {
+    if constexpr (MODE == FW_KV_DENSE) {
+      if (form == kFormMid) {
+        if (d == 64) launch_fr<MODE, 64, 64, 4, 2, 2, 2>(a, grid, s);
+        else if (d == 128) launch_fr<MODE, 128, 128, 4, 2, 2, 2>(a, grid, s);
+        else launch_fr<MODE, 192, 128, 4, 2, 2, 2>(a, grid, s);
+        return;
+      }
+      if (form == kFormSmall) {
+        if (d == 64) launch_fr<MODE, 64, 64, 1, 8, 1, 2>(a, grid, s);
+        else if (d == 128) launch_fr<MODE, 128, 128, 1, 4, 1, 2>(a, grid, s);
+        else launch_fr<MODE, 192, 128, 1, 4, 1, 2>(a, grid, s);
+        return;
+      }
+    }
     if (d == 128 && dv == 128) {
       if constexpr (MODE == FW_KV_DENSE) {
         if (use_pair(a, grid)) {
@@ -2410,8 +2636,7 @@ static void launch_mode(const PrefillArgs &a, dim3 grid, int kv_dtype, int d, in
       if (a.softcap_log2 != 0.f) fw_prefill_d256_kernel<MODE, true><<<grid, 256, 0, s>>>(a);
       else fw_prefill_d256_kernel<MODE, false><<<grid, 256, 0, s>>>(a);
     } else if (d == 64 && dv == 64) {
-      if (a.softcap_log2 != 0.f) fw_prefill_d64_kernel<MODE, true><<<grid, 256, 0, s>>>(a);
-      else fw_prefill_d64_kernel<MODE, false><<<grid, 256, 0, s>>>(a);
+      launch_fr<MODE, 64, 64, 4, 1, 3, 3>(a, grid, s);
     } else if constexpr (MODE == FW_KV_PAGED) {  // pools at 384 and 512: 128-dim V chunks
       if (d == 384) launch_staged<MODE, FW_BF16, 384, 128>(a, grid, s);
       else launch_staged<MODE, FW_BF16, 512, 128>(a, grid, s);
@@ -2421,7 +2646,7 @@ static void launch_mode(const PrefillArgs &a, dim3 grid, int kv_dtype, int d, in
       else if (d == 64) launch_staged<MODE, FW_BF16, 64, 256>(a, grid, s);  // dv 256, or a half of 512
       else if (d == 96) launch_staged<MODE, FW_BF16, 96, 96>(a, grid, s);
       else if (d == 192 && dv == 192) launch_staged<MODE, FW_BF16, 192, 192>(a, grid, s);
-      else if (d == 192) launch_staged<MODE, FW_BF16, 192, 128>(a, grid, s);
+      else if (d == 192) launch_fr<MODE, 192, 128, 4, 1, 2, 2>(a, grid, s);
       else if (d == 384) launch_staged<MODE, FW_BF16, 384, 128>(a, grid, s);
       else launch_staged<MODE, FW_BF16, 512, 128>(a, grid, s);
     }
@@ -2517,13 +2742,14 @@ extern "C" int fw_prefill(const fw_prefill_params *p, fw_stream_t stream) {
   a.G = p->nheads / p->nheads_k;
   a.Sq = p->seqlen_q;
   a.Sk = p->seqlen_k;
-  a.hpw_shift = pp_head_shift(p);
+  const int form = dense_form(p);
+  a.hpw_shift = pp_head_shift(p, form);
   a.vdim0 = 0;
   a.split_max = 0;
   a.split_code = nullptr;
   a.split_cnt = nullptr;
   a.split_part = nullptr;
-  const int qt_rows = prefill_tile_rows(p);
+  const int qt_rows = prefill_tile_rows(p, form);
   const int head_groups = p->nheads >> a.hpw_shift;
   a.n_qt = (p->seqlen_q + qt_rows - 1) / qt_rows;
   a.P = p->page_size;
@@ -2556,7 +2782,7 @@ extern "C" int fw_prefill(const fw_prefill_params *p, fw_stream_t stream) {
     const int w = v_chunk_width(d, dv);
     for (int c = 0; c * w < dv; ++c)
       launch_mode<FW_KV_DENSE>(v_chunk(a, c, w), dim3(a.n_qt * p->batch * head_groups), p->kv_dtype,
-                               p->head_dim, w, s);
+                               p->head_dim, w, s, form);
     return check_launch("fw_prefill");
   }
   FW_REQUIRE(p->cu_seqlens_q && p->workspace, FW_ERR_VALUE, "cu_seqlens_q and workspace required");

@@ -279,9 +279,10 @@ def test_prefill_bitwise_repeat():
 # (docs/v7x.md:49-60, 157-169).
 
 
-# Head dims of q/k and v: the d256 and d64 kernels, the register-staged kernel at 96
-# and 192 and with head_dim_v != head_dim (inputs.py:193-207); the reference's
-# compiled set (test_prefill.py:52,205-208), 384 and 512 (multiples of 128,
+# Head dims of q/k and v: the d256 kernel, the free-running one at 64 and
+# 192/128, the register-staged kernel at 96, 192 and the other head_dim_v !=
+# head_dim (inputs.py:193-207); the reference's compiled set
+# (test_prefill.py:52,205-208), 384 and 512 (multiples of 128,
 # inputs.py:100-140) plus 128/256 and 256/128.  A head_dim_v above 256 runs as
 # launches over chunks of v and out.
 HEAD_DIMS = [(256, 256), (64, 64), (128, 256), (256, 128), (96, 96), (192, 192), (192, 128),
@@ -337,6 +338,41 @@ def test_head_dim_64_tile_edges(g, sq, sk, causal, window, softcap):
                              round_scaled_q=True)
     assert_close(out.float().cpu().numpy(), head_major(ro))
     assert_lse(lse.cpu().numpy(), rl)
+
+
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 128), (192, 128)])
+@pytest.mark.parametrize("b,h,hk,sq,sk,causal,window,softcap", [
+    # one wave per key group and 32 rows (8 key tiles or more)
+    (1, 2, 1, 1, 1100, True, (-1, -1), 0.0),    # more key tiles than groups by one or two
+    (1, 3, 1, 33, 512, True, (-1, -1), 30.0),   # a row past a q tile; group sizes equal
+    (1, 4, 2, 600, 600, True, (-1, -1), 0.0),   # leading q tiles with fewer tiles than groups
+    (1, 2, 2, 600, 520, True, (-1, -1), 0.0),   # rows that see nothing
+    (2, 2, 2, 70, 900, False, (700, 3), 0.0),
+    # two key groups of four waves
+    (1, 4, 1, 65, 130, True, (-1, -1), 0.0),    # three key tiles: the second group has one
+    (3, 24, 6, 129, 700, True, (-1, -1), 0.0),  # 4 heads a workgroup, 11 key tiles
+    (3, 30, 15, 300, 513, False, (-1, -1), 50.0),
+    # up to two such workgroups per CU
+    (1, 20, 20, 2050, 2100, True, (-1, -1), 0.0),
+])
+def test_dense_forms(d, dv, b, h, hk, sq, sk, causal, window, softcap):
+    """Dense calls whose grid leaves CUs idle: the key tiles of a q tile split
+    over waves and merged (dense_form)."""
+    announce(f"dense form d{d}/{dv} b{b} h{h}/{hk} sq{sq} sk{sk} causal={causal} window={window}")
+    rng = np.random.default_rng(72)
+    q, k, v = randn(rng, (b, sq, h, d)), randn(rng, (b, sk, hk, d)), randn(rng, (b, sk, hk, dv))
+    s = rng.standard_normal(h).astype(np.float32) if sq % 2 else None
+    out, lse = flash_attn_func(
+        to_dev_bf16(head_major(q)), to_dev_bf16(head_major(k)), to_dev_bf16(head_major(v)),
+        causal=causal, window_size=window, softcap=softcap, return_softmax_lse=True,
+        learnable_sink=None if s is None else torch.tensor(s, device=DEV))
+    check = slice(0, h) if sq * sk < 1 << 20 else slice(h - 1, h)  # the oracle's time
+    kv = slice(0, hk) if sq * sk < 1 << 20 else slice(hk - 1, hk)
+    ro, rl = A.attention_ref(q[:, :, check], k[:, :, kv], v[:, :, kv], causal=causal,
+                             window_size=window, softcap=softcap,
+                             sinks=None if s is None else s[check], round_scaled_q=True)
+    assert_close(out.float().cpu().numpy()[:, check], head_major(ro))
+    assert_lse(lse.cpu().numpy()[:, check], rl)
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
