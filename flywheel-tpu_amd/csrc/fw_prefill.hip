@@ -16,9 +16,9 @@
 //                              the same on large dense grids, two mirrored q
 //                              tiles per workgroup
 //   fw_prefill_fr_kernel       head dims 64/64 and 192/128 (bf16 K/V), and
-//                              small dense grids at 64, 128 and 192/128:
-//                              free-running waves, the key tiles of a q tile
-//                              split over waves where the grid is small
+//                              smaller calls at 128/128: free-running waves,
+//                              the key tiles of a q tile split over waves
+//                              where a dense grid is small
 //   fw_prefill_staged_kernel   the other head dims (96, 192, 384, 512, mixed
 //                              q / v widths) and fp8 pools at 64: K/V staged
 //                              in registers
@@ -1846,7 +1846,7 @@ __global__ __launch_bounds__(256, 1) void fw_prefill_d256_pair_kernel(PrefillArg
 // registers): 120 us; without the exponentials 66 us, without the copies 69.
 // 192/128, 64/8 heads x 4096 tokens 288 us, 16/16 x 2048 x 3000 62 us and 52 us
 // in the mid form (register-staged: 129).  What the forms are worth on smaller
-// grids stands at dense_form.
+// calls stands at prefill_form.
 constexpr int kFrKeys = 64;
 // 16-byte chunk swizzle of LDS row r: 256-byte rows as in the ping-pong kernel
 // (swz).  Rows of 128 and 384 bytes alternate between the halves of the 64
@@ -2467,17 +2467,21 @@ static bool use_fr(const fw_prefill_params *p) {
                                     (p->head_dim == 192 && head_dim_v_of(p) == 128));
 }
 
-// Forms of a dense call at head dims 64/64, 128/128 and 192/128 by the size of
-// its grid: kFormLarge is the kernel the head dim runs everywhere, the others
-// fw_prefill_fr_kernel with the key tiles of a q tile split over waves.
-constexpr int kFormLarge = 0, kFormMid = 1, kFormSmall = 2;
+// Forms of a call at head dims 64/64, 128/128 and 192/128 by its size:
+// kFormLarge is what the head dim runs on large calls; kFormFree (128/128) and,
+// for small dense grids, kFormMid and kFormSmall are forms of
+// fw_prefill_fr_kernel (four waves; two groups of four; single waves).
+constexpr int kFormLarge = 0, kFormMid = 1, kFormSmall = 2, kFormFree = 3;
 
 // log2 of the query heads per workgroup: the largest power of two that
 // divides the GQA group size (1 for MHA), up to the workgroup's waves that
 // hold different rows (8 in the ping-pong kernel, 4 in fw_prefill_fr_kernel, 1
 // in its small form); the other kernels take one.
-static int pp_head_shift(const fw_prefill_params *p, int form = kFormLarge) {
-  const int most = form == kFormMid ? 2 : form == kFormSmall ? 0 : use_pingpong(p) ? 3 : use_fr(p) ? 2 : 0;
+static int pp_head_shift(const fw_prefill_params *p, int form) {
+  const int most = form == kFormSmall                ? 0
+                   : form != kFormLarge || use_fr(p) ? 2
+                   : use_pingpong(p)                 ? 3
+                                                     : 0;
   const int G = p->nheads_k > 0 ? p->nheads / p->nheads_k : 1;
   int sh = 0;
   while (sh < most && G % (2 << sh) == 0) ++sh;
@@ -2485,13 +2489,13 @@ static int pp_head_shift(const fw_prefill_params *p, int form = kFormLarge) {
 }
 
 // q rows per schedule slot (and per dense q tile).
-static int prefill_tile_rows(const fw_prefill_params *p, int form = kFormLarge) {
+static int prefill_tile_rows(const fw_prefill_params *p, int form) {
   if (form == kFormSmall) return 32;
   return (form == kFormLarge && use_pingpong(p) ? kPPRows : kQT) >> pp_head_shift(p, form);
 }
 
-// The form of a dense call, by the workgroups each would launch on the CUs and
-// the key tiles T a q tile visits.  Measured (us per call, large / mid / small,
+// The form of a call.  Dense: by the workgroups each would launch on the CUs
+// and the key tiles T a q tile visits.  Measured (us per call, large / mid / small,
 // 256 CUs; heads x queries x keys):
 //   small, while one workgroup per 32 rows fits the CUs and T >= 8:
 //     128/128   8/2 x 512 x 512 17.8 / 13.2 / 11.3, 8/2 x 64 x 4096 76 / 49 / 31,
@@ -2500,9 +2504,9 @@ static int prefill_tile_rows(const fw_prefill_params *p, int form = kFormLarge) 
 //               two rounds of workgroups 16/4 x 1024 x 1024 26 / 19 / 23
 //     64/64     8/2 x 512 x 512 10.3 / 9.8 / 8.5, 8/2 x 64 x 4096 50 / 37 / 17
 //     192/128   8/2 x 512 x 512 15.5 / 15.2 / 12.4, 8/2 x 64 x 4096 78 / 58 / 35
-//   mid, while its 128-row workgroups fit the CUs (the other two from T = 8,
-//   where large runs several workgroups per CU):
-//     128/128   16/16 x 2048 x 2048 44.8 / 29.8, 16 x (16/16 x 256 x 256) 15.8 / 11.3
+//   mid, while its 128-row workgroups fit the CUs, from T = 8:
+//     128/128   16/16 x 2048 x 2048 44.8 / 29.8, 16/4 x 700 x 700 21.1 / 15.7
+//               (the four-wave form below: 16.7; T = 5 14.6 / 11.5, 10.6)
 //     64/64     16/16 x 2048 x 2048 28.4 / 21.9, T = 4 8.4 / 8.3
 //     192/128   16/16 x 2048 x 3000 62.1 / 51.9, T = 8 15.6 / 15.5, T = 4 11.3 / 12.1
 //   and up to two workgroups per CU when the causal mask makes long q tiles
@@ -2510,8 +2514,29 @@ static int prefill_tile_rows(const fw_prefill_params *p, int form = kFormLarge) 
 //     128/128   32/32 x 2048 x 2048 49.2 / 41.0 (not causal 58 / 66; 40 heads
 //               56 / 61), 32/8 x 1024 x 1024 twice 28.1 / 27.8
 //     64/64     32/32 x 2048 x 2048 29.3 / 26.6, 192/128 52.3 / 49.9
-static int dense_form(const fw_prefill_params *p) {
-  if (p->kv_mode != FW_KV_DENSE || !(use_fr(p) || use_pingpong(p))) return kFormLarge;
+// At 128/128 the four-wave form (two workgroups per CU, whose prologues and
+// epilogues run beside each other's loops) beats the ping-pong kernel (whose
+// 256 rows a copied tile costs less power) while a query row sees few keys on
+// average, or the ping-pong grid is one round and a bit (us per call, large /
+// free):
+//   below 1,024 keys a row   16 x (32/8 x 1024 x 1024, causal) 171 / 163,
+//     4 x 1536 97.8 / 80.9, 16 x 700 not causal 147 / 137, 8 x 100 11.0 / 8.0;
+//     at 1,024 (8 x 1024, not causal) 132.7 / 133.7, 8 x 2048 causal 269 / 269,
+//     2 x 2048 causal 66 / 71, 32/4 x 4096 not causal 226 / 242
+//   up to three 128-row workgroups per CU and 1,600 keys   40/8 x 2048 causal
+//     56.2 / 48.9, 32/8 x 3000 causal 76.2 / 73.8, 3 x 1024 not causal 57.6 / 51.2
+//   packed sequences, by their mean length (ragged rows even out better in
+//     smaller workgroups): 64 x ~150 91 / 65, 32 x ~500 168 / 142, 16 x ~1035
+//     244 / 230, 16 x ~1900 538 / 526, 16 x ~2120 721 / 745, 4 x ~6000 1101 / 1123
+//   paged rows, whose lengths only the device knows, by the width of the
+//     block table.
+static int prefill_form(const fw_prefill_params *p) {
+  if (!(use_fr(p) || use_pingpong(p))) return kFormLarge;
+  if (p->kv_mode != FW_KV_DENSE) {
+    if (!use_pingpong(p) || p->kv_dtype != FW_BF16 || p->batch <= 0) return kFormLarge;
+    const long keys = p->kv_mode == FW_KV_VARLEN ? p->seqlen_k / p->batch : (long)p->max_pages * p->page_size;
+    return keys <= 1920 ? kFormFree : kFormLarge;
+  }
   const long cus = device_cus();
   auto grid = [&](int form) {
     const int rows = prefill_tile_rows(p, form);
@@ -2523,9 +2548,13 @@ static int dense_form(const fw_prefill_params *p) {
   const long tiles = (keys + kFrKeys - 1) / kFrKeys;
   if (grid(kFormSmall) <= cus && tiles >= 8) return kFormSmall;
   const long mid = grid(kFormMid);
-  if (mid <= cus && (tiles >= 8 || use_pingpong(p))) return kFormMid;
+  if (mid <= cus && tiles >= 8) return kFormMid;
   const bool uneven = p->causal && p->window_left < 0 && 2l * p->seqlen_q >= p->seqlen_k;
   if (mid <= 2 * cus && uneven && tiles >= 32) return kFormMid;
+  if (use_pingpong(p)) {
+    const long mean = p->causal ? std::min(keys, p->seqlen_k - std::min(p->seqlen_q, p->seqlen_k) / 2l) : keys;
+    if (mean < 1024 || (mid <= 3 * cus && mean < 1600)) return kFormFree;
+  }
   return kFormLarge;
 }
 
@@ -2535,10 +2564,10 @@ using namespace fw;
 
 // Key-split pairs the schedule may create (the ping-pong kernel's varlen and
 // paged modes): enough to fill one round of the CUs, at most 32.
-static int split_pairs_max(const fw_prefill_params *p) {
-  if (p->kv_mode == FW_KV_DENSE || !use_pingpong(p)) return 0;
+static int split_pairs_max(const fw_prefill_params *p, int form) {
+  if (p->kv_mode == FW_KV_DENSE || !use_pingpong(p) || form != kFormLarge) return 0;
   if (const char *e = getenv("FW_PREFILL_KEY_SPLIT"); e && e[0] == '0') return 0;
-  const int ng = p->nheads >> pp_head_shift(p);
+  const int ng = p->nheads >> pp_head_shift(p, form);
   return ng > 0 ? std::min(32, std::max(1, 256 / ng)) : 0;
 }
 constexpr size_t kSplitPartBytes = ((size_t)kPPWaves * 32 * 128 + kPPWaves * 32 * 2) * 4;
@@ -2546,10 +2575,10 @@ constexpr size_t kSplitPartBytes = ((size_t)kPPWaves * 32 * 128 + kPPWaves * 32 
 struct PrefillWorkspace {
   size_t sched, codes, cnt, part, total;  // byte offsets of each part, and the size
 };
-static PrefillWorkspace workspace_layout(const fw_prefill_params *p) {
-  const int slots = max_sched_tiles(p, prefill_tile_rows(p)) + split_pairs_max(p);
-  const int sm = split_pairs_max(p);
-  const size_t ng = sm ? (size_t)(p->nheads >> pp_head_shift(p)) : 0;
+static PrefillWorkspace workspace_layout(const fw_prefill_params *p, int form) {
+  const int sm = split_pairs_max(p, form);
+  const int slots = max_sched_tiles(p, prefill_tile_rows(p, form)) + sm;
+  const size_t ng = sm ? (size_t)(p->nheads >> pp_head_shift(p, form)) : 0;
   PrefillWorkspace w;
   w.sched = 0;
   w.codes = align_up((size_t)(1 + 2 * slots) * sizeof(int32_t), 256);
@@ -2561,13 +2590,13 @@ static PrefillWorkspace workspace_layout(const fw_prefill_params *p) {
 
 extern "C" size_t fw_prefill_workspace_bytes(const fw_prefill_params *p) {
   if (p->kv_mode == FW_KV_DENSE) return 0;
-  return workspace_layout(p).total;
+  return workspace_layout(p, prefill_form(p)).total;
 }
 
 // Kernel choice (the host has checked the head dims): 128/128 -> the ping-pong
 // kernel, 256/256 -> the d256 kernel (fp8 pools widened as they land in LDS in
 // both), 64/64 and 192/128 with bf16 K/V -> fw_prefill_fr_kernel (and small
-// dense grids at 128/128: dense_form), everything else (head dims 96, 192/192,
+// dense calls at 128/128: prefill_form), everything else (head dims 96, 192/192,
 // 384, 512, the other head_dim_v != head_dim, fp8 pools at 64) -> the
 // register-staged kernel.  A head_dim_v above 256 runs as
 // launches over chunks of v and out, which keeps O within one wave's
@@ -2597,8 +2626,12 @@ static void launch_fr(const PrefillArgs &a, dim3 grid, hipStream_t s) {
 }
 template <int MODE>
 static void launch_mode(const PrefillArgs &a, dim3 grid, int kv_dtype, int d, int dv,
-                        hipStream_t s, int form = kFormLarge) {
+                        hipStream_t s, int form) {
   if (kv_dtype == FW_BF16) {
+    if (form == kFormFree) {
+      launch_fr<MODE, 128, 128, 4, 1, 2, 2>(a, grid, s);
+      return;
+    }
     if constexpr (MODE == FW_KV_DENSE) {
       if (form == kFormMid) {
         if (d == 64) launch_fr<MODE, 64, 64, 4, 2, 2, 2>(a, grid, s);
@@ -2742,7 +2775,7 @@ extern "C" int fw_prefill(const fw_prefill_params *p, fw_stream_t stream) {
   a.G = p->nheads / p->nheads_k;
   a.Sq = p->seqlen_q;
   a.Sk = p->seqlen_k;
-  const int form = dense_form(p);
+  const int form = prefill_form(p);
   a.hpw_shift = pp_head_shift(p, form);
   a.vdim0 = 0;
   a.split_max = 0;
@@ -2804,9 +2837,9 @@ extern "C" int fw_prefill(const fw_prefill_params *p, fw_stream_t stream) {
   if (p->seqlen_q <= 0) return FW_OK;
   const int max_tiles = max_sched_tiles(p, qt_rows);
   const bool varlen = p->kv_mode == FW_KV_VARLEN;
-  const PrefillWorkspace wl = workspace_layout(p);
+  const PrefillWorkspace wl = workspace_layout(p, form);
   uint8_t *ws = (uint8_t *)p->workspace;
-  a.split_max = split_pairs_max(p);
+  a.split_max = split_pairs_max(p, form);
   a.split_code = a.split_max ? (const int32_t *)(ws + wl.codes) : nullptr;
   a.split_cnt = a.split_max ? (int *)(ws + wl.cnt) : nullptr;
   a.split_part = a.split_max ? (float *)(ws + wl.part) : nullptr;
@@ -2841,11 +2874,11 @@ extern "C" int fw_prefill(const fw_prefill_params *p, fw_stream_t stream) {
   if (p->kv_mode == FW_KV_VARLEN) {
     const int w = v_chunk_width(d, dv);
     for (int c = 0; c * w < dv; ++c)
-      launch_mode<FW_KV_VARLEN>(v_chunk(a, c, w), grid, FW_BF16, p->head_dim, w, s);
+      launch_mode<FW_KV_VARLEN>(v_chunk(a, c, w), grid, FW_BF16, p->head_dim, w, s, form);
   } else {
     const int w = v_chunk_width(d, dv);
     for (int c = 0; c * w < dv; ++c)
-      launch_mode<FW_KV_PAGED>(v_chunk(a, c, w), grid, p->kv_dtype, p->head_dim, w, s);
+      launch_mode<FW_KV_PAGED>(v_chunk(a, c, w), grid, p->kv_dtype, p->head_dim, w, s, form);
   }
   return check_launch("fw_prefill");
 }

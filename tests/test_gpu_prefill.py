@@ -375,6 +375,89 @@ def test_dense_forms(d, dv, b, h, hk, sq, sk, causal, window, softcap):
     assert_lse(lse.cpu().numpy()[:, check], rl)
 
 
+@pytest.mark.parametrize("b,h,hk,sq,sk,causal,window,softcap,sinks", [
+    # the ping-pong kernel (many rows, at least 1,600 keys a row): ragged ends
+    # on both sides, 1, 2 and 8 heads a workgroup
+    (1, 30, 30, 1150, 2305, False, (-1, -1), 0.0, True),
+    (2, 18, 9, 1055, 2113, False, (1800, 700), 50.0, False),
+    (1, 64, 8, 2309, 3457, True, (-1, -1), 0.0, False),
+    # the four-wave form: tile edges, 1, 2 and 4 heads a workgroup
+    (5, 24, 8, 257, 257, True, (-1, -1), 0.0, True),
+    (9, 10, 5, 129, 191, False, (64, 17), 30.0, False),
+    (16, 16, 4, 97, 65, True, (-1, -1), 0.0, False),
+])
+def test_dense_large_and_free_forms(b, h, hk, sq, sk, causal, window, softcap, sinks):
+    announce(f"dense form b{b} h{h}/{hk} sq{sq} sk{sk} causal={causal} window={window}")
+    rng = np.random.default_rng(73)
+    q, k, v = randn(rng, (b, sq, h, 128)), randn(rng, (b, sk, hk, 128)), randn(rng, (b, sk, hk, 128))
+    s = rng.standard_normal(h).astype(np.float32) if sinks else None
+    out, lse = flash_attn_func(
+        to_dev_bf16(head_major(q)), to_dev_bf16(head_major(k)), to_dev_bf16(head_major(v)),
+        causal=causal, window_size=window, softcap=softcap, return_softmax_lse=True,
+        learnable_sink=None if s is None else torch.tensor(s, device=DEV))
+    hs, ks = slice(h - h // hk, h), slice(hk - 1, hk)  # the last KV head's group, last batch
+    ro, rl = A.attention_ref(q[-1:, :, hs], k[-1:, :, ks], v[-1:, :, ks], causal=causal,
+                             window_size=window, softcap=softcap,
+                             sinks=None if s is None else s[hs], round_scaled_q=True)
+    assert_close(out[-1:, hs].float().cpu().numpy(), head_major(ro))
+    assert_lse(lse[-1:, hs].cpu().numpy(), rl)
+
+
+@pytest.mark.parametrize("wide", [False, True])  # the four-wave form, the ping-pong kernel
+@pytest.mark.parametrize("dense_kv", [False, True])
+def test_ragged_forms(wide, dense_kv):
+    """Packed varlen and paged rows on both sides of prefill_form's line (mean
+    length, block-table width), the same sequences on each."""
+    announce(f"ragged forms wide={wide} packed={dense_kv}")
+    rng = np.random.default_rng(74)
+    qlens, prior = [65, 1, 256, 33, 0, 130], [0, 300, 17, 64, 5, 129]
+    h, hk = 8, 2
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(qlens)]), dtype=torch.int32, device=DEV)
+    if not dense_kv:
+        case = PagedCase(rng, batch=6, nheads=h, nheads_k=hk, lengths=prior, new_tokens=qlens,
+                         max_pages=200 if wide else 25)
+        q = randn(rng, (sum(qlens), h, 128))
+        pool = case.pool()
+        out, lse, _ = flash_attn_with_kvcache(
+            to_dev_bf16(q), pool, None, dev_from_codes(case.k_codes, case.dtype),
+            dev_from_codes(case.v_codes, case.dtype),
+            cache_seqlens=torch.tensor(prior, dtype=torch.int32, device=DEV),
+            block_table=torch.tensor(case.table, device=DEV), cu_seqlens_q=cu,
+            max_seqlen_q=max(qlens), causal=True, return_softmax_lse=True)
+        exp = case.expected_pool()
+        np.testing.assert_array_equal(codes_of(pool), exp)
+        krows, vrows = case.rows(exp)
+        out, lse = out.float().cpu().numpy(), lse.cpu().numpy()
+        for i, (n, p) in enumerate(zip(qlens, prior)):
+            if n == 0:
+                continue
+            rows = slice(int(cu[i]), int(cu[i + 1]))
+            ro, rl = A.attention_ref(q[None, rows], krows[None, i, :n + p], vrows[None, i, :n + p],
+                                     causal=True, round_scaled_q=True)
+            assert_close(out[rows], ro[0])
+            assert_lse(lse[:, rows], rl[0])
+        return
+    klens = [n + p for n, p in zip(qlens, prior)]
+    if wide:
+        klens[2] += 12000
+    cuk = np.concatenate([[0], np.cumsum(klens)])
+    q = randn(rng, (sum(qlens), h, 128))
+    k, v = randn(rng, (sum(klens), hk, 128)), randn(rng, (sum(klens), hk, 128))
+    hm = lambda x: to_dev_bf16(x.transpose(1, 0, 2))
+    out, lse = flash_attn_varlen_func(hm(q), hm(k), hm(v), cu,
+                                      torch.tensor(cuk, dtype=torch.int32, device=DEV), max(qlens),
+                                      max(klens), causal=True, return_softmax_lse=True)
+    out, lse = out.float().cpu().numpy(), lse.cpu().numpy()
+    for i, n in enumerate(qlens):
+        if n == 0:
+            continue
+        rows, keys = slice(int(cu[i]), int(cu[i + 1])), slice(int(cuk[i]), int(cuk[i + 1]))
+        ro, rl = A.attention_ref(q[None, rows], k[None, keys], v[None, keys], causal=True,
+                                 round_scaled_q=True)
+        assert_close(out[:, rows], ro[0].transpose(1, 0, 2))
+        assert_lse(lse[:, rows], rl[0])
+
+
 @pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("jump", [40.0, 600.0])
 def test_flash_attn_func_anchor_rescale(d, jump):
