@@ -2297,9 +2297,9 @@ __global__ __launch_bounds__(64 * RW * KG, OCC) void fw_prefill_fr_kernel(Prefil
 
 // One workgroup: per-sequence q tiles from cu_seqlens_q, then padding tiles
 // for the packed rows past cu_seqlens_q[num_active] (schedule.py:617-717).
-// When there are at most kSortTiles sequence tiles they are ordered by cost,
-// the number of 64-key tiles a q tile visits (its causal/window key range),
-// heaviest first, so the longest workgroups start first and the short ones
+// When there are at most kSortTiles sequence tiles they are ordered by cost
+// bucket (the number of 64-key tiles a q tile visits, its causal/window key
+// range), heaviest first, so the longest workgroups start first and the short ones
 // fill the tail (a greedy longest-first list schedule); padding tiles go last.
 // The order changes no result: every q tile is computed independently.
 constexpr int kSortTiles = 2048;
@@ -2324,7 +2324,43 @@ struct SchedArgs {
   int split_max, ng, cus;
 };
 // The schedule, run by one workgroup of blockDim.x threads (a power of two,
-// 64 .. 1024).
+// 64 .. 1024): a thread per tile finds its sequence by binary search over the
+// sequences' first tiles, and a counting sort over cost buckets orders the
+// tiles.  The counts are kept per run of 64 tiles, one wave each, so the order
+// (and with it the choice of split tiles) is the same on every call.  A rank
+// sort (every tile against every other) is quadratic: 540 tiles 12,000 cycles,
+// 2,048 fifteen times that.
+constexpr int kSchedSeqs = 2048;
+constexpr int kCostBuckets = 512;
+// Costs (64-key tiles) to buckets, heaviest first: exact below 64, 32 steps
+// an octave above.
+__device__ __forceinline__ int cost_bucket(int cost) {
+  int c = cost;
+  if (cost >= 64) {
+    const int e = min(31 - __builtin_clz(cost), 19);
+    c = 64 + 32 * (e - 6) + min((cost >> (e - 5)) - 32, 31);
+  }
+  return kCostBuckets - 1 - c;
+}
+// Inclusive scan of v over the workgroup's threads; total = the sum of all.
+// part: 16 ints of LDS (two barriers).
+__device__ __forceinline__ int block_scan(int v, int *part, int &total) {
+  const int tid = threadIdx.x, lane = tid & 63;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int u = __shfl_up(v, d, 64);
+    if (lane >= d) v += u;
+  }
+  __syncthreads();
+  if (lane == 63) part[tid >> 6] = v;
+  __syncthreads();
+  total = 0;
+  for (int i = 0; i < (int)blockDim.x >> 6; ++i) {
+    if (i < tid >> 6) v += part[i];
+    total += part[i];
+  }
+  return v;
+}
 __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
   const int32_t *cu_q = sa.cu_q, *num_active = sa.num_active, *cu_k = sa.cu_k,
                 *seqused_k = sa.seqused_k;
@@ -2333,10 +2369,14 @@ __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
             cus = sa.cus;
   int32_t *sched = sa.sched, *split_code = sa.split_code;
   int *split_cnt = sa.split_cnt;
-  __shared__ int part[1024];
-  __shared__ unsigned long long key[kSortTiles];
-  __shared__ int eseq[kSortTiles], eq0[kSortTiles];
+  __shared__ int part[16];
+  __shared__ uint16_t first[kSchedSeqs];  // a sequence's first tile
+  __shared__ uint16_t seq_of[kSortTiles];
+  __shared__ uint32_t key[kSortTiles];    // bucket << 6 | rank among its run's equals
+  __shared__ __attribute__((aligned(16))) uint16_t cnt[kSortTiles / 64][kCostBuckets];
+  __shared__ int heavier[kCostBuckets];   // tiles in the buckets before
   const int tid = threadIdx.x, nt = blockDim.x;  // nt: a power of two, 64 .. 1024
+  const int lane = tid & 63;
   {
     // one round trip brings every input of a batch up to nt sequences into
     // the caches (the loops below read them in dependent steps)
@@ -2345,81 +2385,110 @@ __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
     const int w2 = tid < B ? (cu_k ? cu_k[tid + 1] : seqused_k[tid]) : 0;
     asm volatile("" ::"v"(w0 + w1 + w2));
   }
+  for (int i = tid; i < split_max * ng; i += nt) split_cnt[i] = 0;
   const int nact = num_active ? min(max(*num_active, 0), B) : B;
   const int per = (nact + nt - 1) / nt;
   const int s0 = tid * per, s1 = min(nact, s0 + per);
   int mine = 0;
   for (int s = s0; s < s1; ++s) mine += (cu_q[s + 1] - cu_q[s] + qt - 1) / qt;
-  part[tid] = mine;
-  __syncthreads();
-  for (int o = 1; o < nt; o <<= 1) {  // inclusive scan
-    int v = tid >= o ? part[tid - o] : 0;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
-  }
-  const int real = part[nt - 1];
-  const bool sort = real <= kSortTiles;
-  int idx = part[tid] - mine;
-  for (int s = s0; s < s1; ++s) {
-    const int len = cu_q[s + 1] - cu_q[s];
-    const int sk = cu_k ? cu_k[s + 1] - cu_k[s] : seqused_k[s] + (plus_q ? len : 0);
-    const int off = sk - len;  // bottom-right alignment, as in the kernels
-    for (int q0 = 0; q0 < len; q0 += qt) {
-      if (sort) {
-        const int last = min(q0 + qt, len) - 1;
-        const int lo = wl >= 0 ? max(0, q0 + off - wl) : 0;
-        const int hi = wr >= 0 ? min(sk, last + off + wr + 1) : sk;
-        const int cost = hi > lo ? (hi + kKT - 1) / kKT - lo / kKT : 0;
-        key[idx] = ((unsigned long long)cost << 32) | (unsigned)(idx + 1);
-        eseq[idx] = s;
-        eq0[idx] = q0;
-      } else if (idx < max_tiles) {
-        sched[1 + 2 * idx] = s;
-        sched[2 + 2 * idx] = q0;
-        if (split_max > 0) split_code[idx] = -1;
-      }
-      ++idx;
-    }
-  }
+  int real;
+  int idx = block_scan(mine, part, real) - mine;
+  const bool sort = real <= kSortTiles && nact <= kSchedSeqs;
+  const int cap = max_tiles + split_max;  // schedule slots
   int nsplit = 0;  // the nsplit heaviest tiles are split (ranks 0 .. nsplit - 1)
-  if (sort && split_max > 0) {
-    __shared__ int nbig;
-    if (tid == 0) nbig = 0;
-    for (int i = tid; i < split_max * ng; i += nt) split_cnt[i] = 0;
+  if (!sort) {  // sequence order
+    for (int s = s0; s < s1; ++s) {
+      const int len = cu_q[s + 1] - cu_q[s];
+      for (int q0 = 0; q0 < len; q0 += qt, ++idx)
+        if (idx < max_tiles) {
+          sched[1 + 2 * idx] = s;
+          sched[2 + 2 * idx] = q0;
+          if (split_max > 0) split_code[idx] = -1;
+        }
+    }
+  } else {
+    for (int s = s0; s < s1; ++s) {
+      first[s] = (uint16_t)idx;
+      idx += (cu_q[s + 1] - cu_q[s] + qt - 1) / qt;
+    }
+    const int runs = (real + 63) / 64;
+    for (int i = tid; i < runs * kCostBuckets / 8; i += nt)
+      ((u32x4_t *)&cnt[0][0])[i] = u32x4_t{0, 0, 0, 0};
     __syncthreads();
-    int mybig = 0;
-    for (int i = tid; i < real; i += nt) mybig += (int)(key[i] >> 32) >= kMinSplitCost;
-    if (mybig) atomicAdd(&nbig, mybig);
+    for (int r = tid >> 6; r < runs; r += nt >> 6) {
+      const int i = 64 * r + lane;
+      int lo = 0, bucket = 0;
+      if (i < real) {
+        // the last sequence starting at or before tile i (sequences without
+        // rows share their successor's first tile)
+        int hi = nact;
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if ((int)first[mid] <= i) lo = mid; else hi = mid;
+        }
+        const int len = cu_q[lo + 1] - cu_q[lo];
+        const int sk = cu_k ? cu_k[lo + 1] - cu_k[lo] : seqused_k[lo] + (plus_q ? len : 0);
+        const int off = sk - len;  // bottom-right alignment, as in the kernels
+        const int q0 = (i - first[lo]) * qt, last = min(q0 + qt, len) - 1;
+        const int k_lo = wl >= 0 ? max(0, q0 + off - wl) : 0;
+        const int k_hi = wr >= 0 ? min(sk, last + off + wr + 1) : sk;
+        bucket = cost_bucket(k_hi > k_lo ? (k_hi + kKT - 1) / kKT - k_lo / kKT : 0);
+      }
+      // the run's tiles of the same bucket, one bit each
+      uint64_t same = __ballot(i < real);
+#pragma unroll
+      for (int bit = 0; bit < 9; ++bit) {
+        const uint64_t set = __ballot((bucket >> bit) & 1);
+        same &= (bucket >> bit) & 1 ? set : ~set;
+      }
+      if (i < real) {
+        const int before = __popcll(same & ((1ull << lane) - 1));
+        seq_of[i] = (uint16_t)lo;
+        key[i] = (uint32_t)bucket << 6 | before;
+        if (before == 0) cnt[r][bucket] = (uint16_t)__popcll(same);
+      }
+    }
+    __syncthreads();
+    // cnt[r][bucket]: the bucket's tiles in earlier runs; then the buckets' sums
+    const int bpt = max(1, kCostBuckets / nt);  // buckets per thread
+    int sum = 0;
+    if (tid * bpt < kCostBuckets)
+      for (int bk = tid * bpt; bk < (tid + 1) * bpt; ++bk) {
+        heavier[bk] = sum;
+        int run = 0;
+        for (int r = 0; r < runs; ++r) {
+          const int c = cnt[r][bk];
+          cnt[r][bk] = (uint16_t)run;
+          run += c;
+        }
+        sum += run;
+      }
+    int all;
+    const int before = block_scan(sum, part, all) - sum;
+    if (tid * bpt < kCostBuckets)
+      for (int bk = tid * bpt; bk < (tid + 1) * bpt; ++bk) heavier[bk] += before;
     __syncthreads();
     const long wgs = (long)real * ng;
-    if (wgs < 16l * cus) {
+    if (split_max > 0 && wgs < 16l * cus) {
       const int gap = (int)((cus - wgs % cus) % cus);
-      nsplit = min(min(split_max, nbig), (gap + ng - 1) / ng);
+      // tiles of at least kMinSplitCost key tiles
+      const int big = heavier[cost_bucket(kMinSplitCost - 1)];
+      nsplit = min(min(split_max, big), (gap + ng - 1) / ng);
     }
-  }
-  const int cap = max_tiles + split_max;  // schedule slots
-  if (sort) {
-    // Rank sort, descending: a tile's slot is the number of larger keys (keys
-    // are distinct: the low word is the tile's index).  Every thread reads
-    // the same key at the same time (an LDS broadcast), so one pass over the
-    // keys replaces the log^2 barrier-separated stages of a sorting network.
-    __syncthreads();
     for (int i = tid; i < real; i += nt) {
-      const unsigned long long x = key[i];
-      int rank = 0;
-      for (int j = 0; j < real; ++j) rank += key[j] > x;
+      const int bucket = key[i] >> 6, s = seq_of[i], q0 = (i - first[s]) * qt;
+      const int rank = heavier[bucket] + cnt[i >> 6][bucket] + (key[i] & 63);
       // ranks below nsplit all hold tiles of >= kMinSplitCost key tiles
       const bool split = rank < nsplit;
       if (rank < cap) {
-        sched[1 + 2 * rank] = eseq[i];
-        sched[2 + 2 * rank] = eq0[i];
+        sched[1 + 2 * rank] = s;
+        sched[2 + 2 * rank] = q0;
         if (split_max > 0) split_code[rank] = split ? 2 * rank : -1;
       }
       if (split) {  // the second half's slot
         const int r2 = real + rank;
-        sched[1 + 2 * r2] = eseq[i];
-        sched[2 + 2 * r2] = eq0[i];
+        sched[1 + 2 * r2] = s;
+        sched[2 + 2 * r2] = q0;
         split_code[r2] = 2 * rank + 1;
       }
     }
@@ -2447,8 +2516,10 @@ __global__ __launch_bounds__(256) void fw_append_schedule_kernel(AppendArgs ap, 
   else append_token_rows(ap, blockIdx.x - 1);
 }
 
+// Most schedule slots of a call: every sequence and the padding rows end with
+// at most one partly filled tile, and together they hold seqlen_q rows.
 static int max_sched_tiles(const fw_prefill_params *p, int qt) {
-  return 2 * ((p->seqlen_q + qt - 1) / qt) + p->batch + 1;
+  return (p->seqlen_q + qt - 1) / qt + p->batch + 1;
 }
 
 // The ping-pong kernel takes head dim 128 (bf16, or an fp8 pool); its softcap
@@ -2860,10 +2931,9 @@ extern "C" int fw_prefill(const fw_prefill_params *p, fw_stream_t stream) {
     fw_append_schedule_kernel<<<1 + append_blocks(p->seqlen_q), 256, 0, s>>>(ap, sa);
     st = check_launch("fw_append_schedule_kernel");
   } else {
-    // a thread per sequence and per q tile (up to 1024): the rank sort's pass
+    // a thread per sequence and per q tile (up to 1024)
     int sched_threads = 64;
-    while (sched_threads < 1024 &&
-           (sched_threads < p->batch || sched_threads < std::min(max_tiles, kSortTiles)))
+    while (sched_threads < 1024 && (sched_threads < p->batch || sched_threads < 2 * max_tiles))
       sched_threads <<= 1;
     fw_prefill_schedule<<<1, sched_threads, 0, s>>>(sa);
     st = check_launch("fw_prefill_schedule");

@@ -403,6 +403,54 @@ def test_dense_large_and_free_forms(b, h, hk, sq, sk, causal, window, softcap, s
     assert_lse(lse[-1:, hs].cpu().numpy(), rl)
 
 
+def schedule_of(qlens, klens, h, hk, causal, num_rows):
+    """The (sequence, first row) pairs fw_prefill's schedule holds for packed
+    sequences (head dim 128), read back from the workspace."""
+    from flywheel_tpu import _native as N
+    dev = lambda x: torch.tensor(np.concatenate([[0], np.cumsum(x)]), dtype=torch.int32, device=DEV)
+    cu_q, cu_k = dev(qlens), dev(klens)
+    q = torch.zeros((h, num_rows, 128), dtype=torch.bfloat16, device=DEV)
+    k = torch.zeros((hk, max(1, sum(klens)), 128), dtype=torch.bfloat16, device=DEV)
+    out = torch.empty_like(q)
+    p = N.PrefillParams()
+    p.kv_mode, p.q, p.out, p.k, p.v = N.FW_KV_VARLEN, N.ptr(q), N.ptr(out), N.ptr(k), N.ptr(k)
+    p.cu_seqlens_q, p.cu_seqlens_k = N.ptr(cu_q), N.ptr(cu_k)
+    for x, t in (("q", q), ("o", q), ("k", k), ("v", k)):
+        setattr(p, x + "_stride_h", t.shape[1] * 128)
+        setattr(p, x + "_stride_t", 128)
+    p.batch, p.nheads, p.nheads_k, p.head_dim = len(qlens), h, hk, 128
+    p.seqlen_q, p.seqlen_k, p.max_seqlen_q = num_rows, sum(klens), max(qlens)
+    p.kv_dtype, p.softmax_scale, p.causal = N.FW_BF16, 0.1, int(causal)
+    p.window_left = p.window_right = -1
+    p.k_descale = p.v_descale = 1.0
+    ws = torch.zeros(N.lib().fw_prefill_workspace_bytes(p), dtype=torch.uint8, device=DEV)
+    p.workspace, p.workspace_bytes = N.ptr(ws), ws.numel()
+    N.check(N.lib().fw_prefill(p, N.stream_of(q)))
+    w = ws[:ws.numel() // 4 * 4].view(torch.int32).cpu().numpy()
+    return [(int(w[1 + 2 * i]), int(w[2 + 2 * i])) for i in range(w[0])]
+
+
+@pytest.mark.parametrize("n,lo,hi,extra", [
+    (1, 1, 1, 0), (70, 0, 90, 0), (64, 64, 64, 33),
+    (40, 300, 1700, 0),    # ~1,250 tiles of 32 rows: 20 runs of 64
+    (1500, 0, 40, 100),    # more sequences than threads
+    (45, 1800, 2000, 0),   # more than 2,048 tiles: sequence order
+    (2100, 0, 3, 0),       # more than 2,048 sequences: sequence order
+])
+def test_schedule_order(n, lo, hi, extra):
+    """Every tile once, heaviest first, equal costs in sequence order."""
+    announce(f"schedule n{n} {lo}..{hi} + {extra}")
+    rng = np.random.default_rng(75)
+    lens = [int(x) for x in rng.integers(lo, hi + 1, n)]
+    rows = sum(lens)
+    got = schedule_of(lens, lens, 4, 1, True, rows + extra)  # 4 heads of 32 rows
+    tiles = [(s, r) for s in range(n) for r in range(0, lens[s], 32)]
+    if n <= 2048 and len(tiles) <= 2048:
+        # exact buckets below 64 key tiles, the longest here 32
+        tiles.sort(key=lambda t: -min(t[1] + 32, lens[t[0]]) // 64)  # -ceil(keys / 64)
+    assert got == tiles + [(-1, r) for r in range(rows, rows + extra, 32)]
+
+
 @pytest.mark.parametrize("wide", [False, True])  # the four-wave form, the ping-pong kernel
 @pytest.mark.parametrize("dense_kv", [False, True])
 def test_ragged_forms(wide, dense_kv):
