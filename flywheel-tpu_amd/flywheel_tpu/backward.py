@@ -96,6 +96,8 @@ class FlashAttnFunction(torch.autograd.Function):
         ctx.spec = spec
         ctx.save_for_backward(q, k, v, out, lse)
         ctx.mark_non_differentiable(lse)
+        # no zeros in the place of lse's missing gradient (a fill launch a call)
+        ctx.set_materialize_grads(False)
         return out, lse
 
     @staticmethod
@@ -106,7 +108,7 @@ class FlashAttnFunction(torch.autograd.Function):
         q, k, v, out, lse = ctx.saved_tensors
         g = dict(spec["geometry"])
         d, dv = g["head_dim"], g["head_dim_v"]
-        dout, grads = dout.contiguous(), None
+        dout, grads = torch.zeros_like(out) if dout is None else dout.contiguous(), None
         if (d, dv) == (64, 64) or bwd_widths(d, dv) == (d, dv):
             grads = attn_bwd(q, k, v, out, dout, lse, **g)
         if grads is None:

@@ -488,7 +488,8 @@ def flash_attn_varlen_func(
     tables = R.check_tables(rotary_cos, rotary_sin, head_dim=d, dtype=q.dtype,
                             rotate_k=rotary_k, interleaved=rotary_interleaved,
                             kv_len_bound=int(max_seqlen_k))
-    if tables is not None:
+    if tables is not None and not (cu_q.is_cuda or cu_k.is_cuda):
+        # lengths on the device are not read: no launches for the differences
         R.check_packed_lengths(cu_q, torch.diff(cu_k.to(torch.int64)), tables[0].shape[0])
     _check_bf16(q, k, v)
     N.require_device(q, k, v)
