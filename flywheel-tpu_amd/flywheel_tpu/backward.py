@@ -140,5 +140,8 @@ def forward_only(run, msg, q, k, v):
 
 
 def needs_grad(*tensors):
-    return torch.is_grad_enabled() and any(
-        isinstance(t, torch.Tensor) and t.requires_grad for t in tensors)
+    if torch.is_grad_enabled():
+        for t in tensors:
+            if isinstance(t, torch.Tensor) and t.requires_grad:
+                return True
+    return False

@@ -77,19 +77,14 @@ def decode_params(q, kv_cache, k_new, v_new, cache_seqlens, block_table, num_act
     out = torch.empty_like(q)
     lse = (torch.empty((batch, nheads, seqlen_q), dtype=torch.float32, device=q.device)
            if return_lse else None)
-    p = N.DecodeParams()
-    p.q, p.kv_cache, p.k_new, p.v_new = N.ptr(q), N.ptr(kv_cache), N.ptr(k_new), N.ptr(v_new)
-    p.v_cache = N.ptr(v_cache)
-    p.cache_seqlens, p.block_table = N.ptr(cache_seqlens), N.ptr(block_table)
-    p.num_active, p.sinks, p.out, p.lse = N.ptr(num_active), N.ptr(sinks), N.ptr(out), N.ptr(lse)
-    p.batch, p.seqlen_q, p.nheads, p.nheads_k, p.head_dim = batch, seqlen_q, nheads, nheads_k, head_dim
-    p.page_size, p.num_pages, p.max_pages = kv_cache.shape[1], kv_cache.shape[0], block_table.shape[1]
-    p.kv_dtype = N.KV_DTYPES[kv_cache.dtype]
-    p.seqlen_add = seqlen_add
-    p.softmax_scale, p.softcap = softmax_scale, softcap
-    p.causal, p.window_left = int(causal), window_left
+    ptr = N.ptr
+    p = N.DecodeParams(  # in field order: one call, not an attribute at a time
+        ptr(q), ptr(kv_cache), ptr(k_new), ptr(v_new), ptr(cache_seqlens), ptr(block_table),
+        ptr(num_active), ptr(sinks), ptr(out), ptr(lse), None, 0,
+        batch, seqlen_q, nheads, nheads_k, head_dim, kv_cache.shape[1], kv_cache.shape[0],
+        block_table.shape[1], N.KV_DTYPES[kv_cache.dtype], seqlen_add, softmax_scale, softcap,
+        int(causal), window_left, 1.0, 1.0, num_splits, ptr(v_cache))
     keep = set_descales(p, k_descale, v_descale)
-    p.num_splits = num_splits
     return p, out, lse, keep
 
 
@@ -136,23 +131,18 @@ def paged_prefill(q, kv_cache, cu_seqlens_q, seqused_k, block_table, num_active,
     lse = (torch.empty((nheads, total_q), dtype=torch.float32, device=q.device)
            if return_lse else None)
     left, right = effective_window(causal, window_size)
-    p = N.PrefillParams()
-    p.kv_mode = N.FW_KV_PAGED
-    p.q, p.out, p.lse, p.k, p.v = N.ptr(q), N.ptr(out), N.ptr(lse), N.ptr(kv_cache), None
-    p.cu_seqlens_q, p.seqused_k, p.block_table = N.ptr(cu_seqlens_q), N.ptr(seqused_k), N.ptr(block_table)
-    p.num_active, p.sinks = N.ptr(num_active), N.ptr(sinks)
-    p.q_stride_b, p.q_stride_h, p.q_stride_t = 0, qs_h, qs_t
-    p.o_stride_b, p.o_stride_h, p.o_stride_t = 0, qs_h, qs_t
-    p.lse_stride_b, p.lse_stride_h = 0, total_q
-    p.batch, p.nheads, p.nheads_k, p.head_dim = cu_seqlens_q.shape[0] - 1, nheads, nheads_k, head_dim
-    p.seqlen_q, p.seqlen_k, p.max_seqlen_q = total_q, 0, max_seqlen_q
-    p.page_size, p.num_pages, p.max_pages = kv_cache.shape[1], kv_cache.shape[0], block_table.shape[1]
-    p.kv_dtype = N.KV_DTYPES[kv_cache.dtype]
-    p.softmax_scale, p.softcap = softmax_scale, softcap
-    p.causal, p.window_left, p.window_right = int(causal), left, right
+    ptr = N.ptr
+    p = N.PrefillParams(  # in field order
+        N.FW_KV_PAGED, ptr(q), ptr(out), ptr(lse), ptr(kv_cache), None,
+        ptr(cu_seqlens_q), None, ptr(seqused_k), ptr(block_table), ptr(num_active), ptr(sinks),
+        None, 0,
+        0, qs_h, qs_t, 0, qs_h, qs_t, 0, 0, 0, 0, 0, 0, 0, total_q,
+        cu_seqlens_q.shape[0] - 1, nheads, nheads_k, head_dim, total_q, 0, max_seqlen_q,
+        kv_cache.shape[1], kv_cache.shape[0], block_table.shape[1], N.KV_DTYPES[kv_cache.dtype],
+        softmax_scale, softcap, int(causal), left, right)
     keep_d = set_descales(p, k_descale, v_descale)
     p.seqused_k_excludes_q = int(seqused_excludes_q)
-    p.k_new, p.v_new = N.ptr(k_new), N.ptr(v_new)
+    p.k_new, p.v_new = ptr(k_new), ptr(v_new)
     keep = None if q_rotary is None else R.set_q_rotary(p, *q_rotary, q.device)
     lib = N.lib()
     nbytes = lib.fw_prefill_workspace_bytes(p)
@@ -348,7 +338,7 @@ def flash_attn_with_kvcache(
     else:
         is_folded = False
     if is_paged:
-        table = block_table.to(device=device, dtype=torch.int32).contiguous()
+        table = int32_device(block_table, device, "block_table")
     elif cache_batch_idx is None:
         table = torch.arange(batch, dtype=torch.int32, device=device).reshape(batch, 1)
     else:

@@ -125,9 +125,10 @@ def int32_device(x, device, name, shape=None):
         t = torch.tensor([x], dtype=torch.int32, device=device)
     else:
         t = as_tensor(x)
-        if t.is_floating_point() or t.dtype == torch.bool:
-            raise ValueError(f"{name} must be an integer array; got {t.dtype}.")
-        t = t.to(device=device, dtype=torch.int32).contiguous()
+        if t.dtype != torch.int32 or t.device != device or not t.is_contiguous():
+            if t.is_floating_point() or t.dtype == torch.bool:
+                raise ValueError(f"{name} must be an integer array; got {t.dtype}.")
+            t = t.to(device=device, dtype=torch.int32).contiguous()
     if shape is not None and tuple(t.shape) != tuple(shape):
         raise ValueError(f"{name} must be {tuple(shape)}; got {tuple(t.shape)}.")
     return t

@@ -49,25 +49,16 @@ def _run_prefill(mode, q, k, v, out, lse, *, qs, ks, vs, os_, ls, batch, nheads,
                  head_dim, seqlen_q, seqlen_k, causal, window_size, softmax_scale, softcap,
                  sinks, cu_q=None, cu_k=None, max_seqlen_q=0, q_rotary=None, head_dim_v=0):
     left, right = effective_window(causal, window_size)
-    p = N.PrefillParams()
-    p.kv_mode = mode
-    p.q, p.out, p.lse, p.k, p.v = N.ptr(q), N.ptr(out), N.ptr(lse), N.ptr(k), N.ptr(v)
-    p.cu_seqlens_q, p.cu_seqlens_k, p.sinks = N.ptr(cu_q), N.ptr(cu_k), N.ptr(sinks)
-    p.q_stride_b, p.q_stride_h, p.q_stride_t = qs
-    p.k_stride_b, p.k_stride_h, p.k_stride_t = ks
-    p.v_stride_b, p.v_stride_h, p.v_stride_t = vs
-    p.o_stride_b, p.o_stride_h, p.o_stride_t = os_
-    p.lse_stride_b, p.lse_stride_h = ls
-    p.batch, p.nheads, p.nheads_k, p.head_dim = batch, nheads, nheads_k, head_dim
+    ptr = N.ptr
+    p = N.PrefillParams(  # in field order: one call, not an attribute at a time
+        mode, ptr(q), ptr(out), ptr(lse), ptr(k), ptr(v), ptr(cu_q), ptr(cu_k), None, None, None,
+        ptr(sinks), None, 0, *qs, *os_, *ks, *vs, *ls, batch, nheads, nheads_k, head_dim,
+        seqlen_q, seqlen_k, max_seqlen_q, 0, 0, 0, N.FW_BF16, softmax_scale, float(softcap),
+        int(causal), left, right, 1.0, 1.0)
     p.head_dim_v = head_dim_v
-    p.seqlen_q, p.seqlen_k, p.max_seqlen_q = seqlen_q, seqlen_k, max_seqlen_q
-    p.kv_dtype = N.FW_BF16
-    p.softmax_scale, p.softcap = softmax_scale, float(softcap)
-    p.causal, p.window_left, p.window_right = int(causal), left, right
-    p.k_descale, p.v_descale = 1.0, 1.0
     keep = None if q_rotary is None else R.set_q_rotary(p, *q_rotary, q.device)
     lib = N.lib()
-    nbytes = lib.fw_prefill_workspace_bytes(p)
+    nbytes = 0 if mode == N.FW_KV_DENSE else lib.fw_prefill_workspace_bytes(p)
     ws = None
     if nbytes:
         ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
