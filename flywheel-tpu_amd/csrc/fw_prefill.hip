@@ -2542,17 +2542,37 @@ static bool use_fr(const fw_prefill_params *p) {
 // kFormLarge is what the head dim runs on large calls; kFormFree (128/128) and,
 // for small dense grids, kFormMid and kFormSmall are forms of
 // fw_prefill_fr_kernel (four waves; two groups of four; single waves).
-constexpr int kFormLarge = 0, kFormMid = 1, kFormSmall = 2, kFormFree = 3;
+// kFormGeneral is the register-staged kernel, for K/V that the copying kernels
+// cannot address.
+constexpr int kFormLarge = 0, kFormMid = 1, kFormSmall = 2, kFormFree = 3, kFormGeneral = 4;
+
+// The copying kernels (head dims 64/64, 128/128, 192/128, 256/256) form a row's
+// offset inside a copy as a 24-bit product, row * byte stride, so a token
+// stride is at most 16 MiB and not negative.
+static bool row_stride_ok(int64_t st) { return st >= 0 && st < (int64_t)1 << 23; }
+static bool needs_general(const fw_prefill_params *p) {
+  const int d = p->head_dim, dv = head_dim_v_of(p);
+  const bool fr = (d == 64 && dv == 64) || (d == 192 && dv == 128);
+  if (p->kv_dtype != FW_BF16 || !(fr || (d == dv && (d == 128 || d == 256)))) return false;
+  if (p->kv_mode == FW_KV_PAGED)
+    return d == 64 && (((uintptr_t)p->k & 15) != 0 || !row_stride_ok((int64_t)d * merged_heads(p->nheads_k, FW_BF16)));
+  if (!row_stride_ok(p->k_stride_t) || !row_stride_ok(p->v_stride_t)) return true;
+  // 64/64 and 192/128 also copy only rows that start at multiples of 16 bytes;
+  // other rows run the staged kernel's plain vector loads
+  return fr && ((((uintptr_t)p->k | (uintptr_t)p->v) & 15) != 0 ||
+                ((p->k_stride_b | p->k_stride_h | p->k_stride_t | p->v_stride_b | p->v_stride_h |
+                  p->v_stride_t) & 7) != 0);
+}
 
 // log2 of the query heads per workgroup: the largest power of two that
 // divides the GQA group size (1 for MHA), up to the workgroup's waves that
 // hold different rows (8 in the ping-pong kernel, 4 in fw_prefill_fr_kernel, 1
 // in its small form); the other kernels take one.
 static int pp_head_shift(const fw_prefill_params *p, int form) {
-  const int most = form == kFormSmall                ? 0
-                   : form != kFormLarge || use_fr(p) ? 2
-                   : use_pingpong(p)                 ? 3
-                                                     : 0;
+  const int most = form == kFormSmall || form == kFormGeneral ? 0
+                   : form != kFormLarge || use_fr(p)          ? 2
+                   : use_pingpong(p)                          ? 3
+                                                              : 0;
   const int G = p->nheads_k > 0 ? p->nheads / p->nheads_k : 1;
   int sh = 0;
   while (sh < most && G % (2 << sh) == 0) ++sh;
@@ -2601,7 +2621,7 @@ static int prefill_tile_rows(const fw_prefill_params *p, int form) {
 //     244 / 230, 16 x ~1900 538 / 526, 16 x ~2120 721 / 745, 4 x ~6000 1101 / 1123
 //   paged rows, whose lengths only the device knows, by the width of the
 //     block table.
-static int prefill_form(const fw_prefill_params *p) {
+static int form_by_size(const fw_prefill_params *p) {
   if (!(use_fr(p) || use_pingpong(p))) return kFormLarge;
   if (p->kv_mode != FW_KV_DENSE) {
     if (!use_pingpong(p) || p->kv_dtype != FW_BF16 || p->batch <= 0) return kFormLarge;
@@ -2627,6 +2647,9 @@ static int prefill_form(const fw_prefill_params *p) {
     if (mean < 1024 || (mid <= 3 * cus && mean < 1600)) return kFormFree;
   }
   return kFormLarge;
+}
+static int prefill_form(const fw_prefill_params *p) {
+  return needs_general(p) ? kFormGeneral : form_by_size(p);
 }
 
 }  // namespace fw
@@ -2661,18 +2684,24 @@ static PrefillWorkspace workspace_layout(const fw_prefill_params *p, int form) {
 
 extern "C" size_t fw_prefill_workspace_bytes(const fw_prefill_params *p) {
   if (p->kv_mode == FW_KV_DENSE) return 0;
-  return workspace_layout(p, prefill_form(p)).total;
+  // the same bytes whatever K's and V's addresses and strides (a caller may
+  // ask before it has them)
+  return std::max(workspace_layout(p, form_by_size(p)).total, workspace_layout(p, kFormGeneral).total);
 }
+
+extern "C" int fw_prefill_form(const fw_prefill_params *p) { return prefill_form(p); }
 
 // Kernel choice (the host has checked the head dims): 128/128 -> the ping-pong
 // kernel, 256/256 -> the d256 kernel (fp8 pools widened as they land in LDS in
 // both), 64/64 and 192/128 with bf16 K/V -> fw_prefill_fr_kernel (and small
 // dense calls at 128/128: prefill_form), everything else (head dims 96, 192/192,
-// 384, 512, the other head_dim_v != head_dim, fp8 pools at 64) -> the
-// register-staged kernel.  A head_dim_v above 256 runs as
+// 384, 512, the other head_dim_v != head_dim, fp8 pools at 64, and K/V rows
+// the copying kernels cannot address: needs_general) -> the register-staged
+// kernel.  A head_dim_v above 256 runs as
 // launches over chunks of v and out, which keeps O within one wave's
 // registers: 256 dims each at head dim 64, 128 each at head dims 384 and 512
-// (whose Q^T operand alone takes 96-128 registers).
+// (whose Q^T operand alone takes 96-128 registers); so does 256/256 in the
+// register-staged kernel.
 // The dense ping-pong and head_dim-256 kernels run as pairs of q tiles
 // (fw_prefill_pp_pair_kernel, fw_prefill_d256_pair_kernel) when the q tiles
 // pair up and half the grid still covers every CU.
@@ -2699,6 +2728,17 @@ template <int MODE>
 static void launch_mode(const PrefillArgs &a, dim3 grid, int kv_dtype, int d, int dv,
                         hipStream_t s, int form) {
   if (kv_dtype == FW_BF16) {
+    if (form == kFormGeneral) {
+      if constexpr (MODE == FW_KV_PAGED) {
+        launch_staged<MODE, FW_BF16, 64, 64>(a, grid, s);
+      } else {
+        if (d == 64) launch_staged<MODE, FW_BF16, 64, 64>(a, grid, s);
+        else if (d == 128) launch_staged<MODE, FW_BF16, 128, 128>(a, grid, s);
+        else if (d == 192) launch_staged<MODE, FW_BF16, 192, 128>(a, grid, s);
+        else launch_staged<MODE, FW_BF16, 256, 128>(a, grid, s);  // halves of v and out
+      }
+      return;
+    }
     if (form == kFormFree) {
       launch_fr<MODE, 128, 128, 4, 1, 2, 2>(a, grid, s);
       return;
@@ -2788,7 +2828,10 @@ static PrefillArgs v_chunk(PrefillArgs a, int c, int w) {
   return a;
 }
 // Width of those chunks: 256 at head dim 64, else 128 (or dv itself up to 256).
-static int v_chunk_width(int d, int dv) { return dv <= 256 ? dv : d == 64 ? 256 : 128; }
+static int v_chunk_width(int d, int dv, int form) {
+  if (form == kFormGeneral && dv == 256) return 128;
+  return dv <= 256 ? dv : d == 64 ? 256 : 128;
+}
 
 extern "C" int fw_prefill(const fw_prefill_params *p, fw_stream_t stream) {
   const int dv = head_dim_v_of(p);
@@ -2883,7 +2926,7 @@ extern "C" int fw_prefill(const fw_prefill_params *p, fw_stream_t stream) {
     FW_REQUIRE(p->batch > 0 && p->seqlen_q > 0 && p->seqlen_k > 0, FW_ERR_VALUE,
                "batch, seqlen_q and seqlen_k must be positive");
     FW_REQUIRE(p->v, FW_ERR_VALUE, "dense attention needs v");
-    const int w = v_chunk_width(d, dv);
+    const int w = v_chunk_width(d, dv, form);
     for (int c = 0; c * w < dv; ++c)
       launch_mode<FW_KV_DENSE>(v_chunk(a, c, w), dim3(a.n_qt * p->batch * head_groups), p->kv_dtype,
                                p->head_dim, w, s, form);
@@ -2901,6 +2944,9 @@ extern "C" int fw_prefill(const fw_prefill_params *p, fw_stream_t stream) {
     // the kernels read keys in 8- and 16-row groups that never straddle a page
     FW_REQUIRE(p->page_size % 16 == 0, FW_ERR_VALUE,
                "page_size must be a multiple of 16; got %d", p->page_size);
+    // (at head dim 64 such pools run the staged kernel: needs_general)
+    FW_REQUIRE((d != 128 && d != 256) || a.CH < (1 << 24) / (d * dtype_bytes(p->kv_dtype)),
+               FW_ERR_VALUE, "a pool's token row of %d heads x %d is 16 MiB or more", a.CH, d);
   }
   FW_REQUIRE(!p->k_new || (p->kv_mode == FW_KV_PAGED && p->v_new && p->seqused_k_excludes_q),
              FW_ERR_VALUE,
@@ -2942,11 +2988,11 @@ extern "C" int fw_prefill(const fw_prefill_params *p, fw_stream_t stream) {
   // one workgroup per (schedule slot, head group); see sched_slot
   dim3 grid((max_tiles + a.split_max) * head_groups);
   if (p->kv_mode == FW_KV_VARLEN) {
-    const int w = v_chunk_width(d, dv);
+    const int w = v_chunk_width(d, dv, form);
     for (int c = 0; c * w < dv; ++c)
       launch_mode<FW_KV_VARLEN>(v_chunk(a, c, w), grid, FW_BF16, p->head_dim, w, s, form);
   } else {
-    const int w = v_chunk_width(d, dv);
+    const int w = v_chunk_width(d, dv, form);
     for (int c = 0; c * w < dv; ++c)
       launch_mode<FW_KV_PAGED>(v_chunk(a, c, w), grid, p->kv_dtype, p->head_dim, w, s, form);
   }

@@ -18,6 +18,7 @@ _lib = None
 
 FW_OK, FW_ERR_VALUE, FW_ERR_NOT_IMPLEMENTED, FW_ERR_RUNTIME = 0, 1, 2, 3
 FW_BF16, FW_FP8_E4M3, FW_FP8_E5M2 = 0, 1, 2
+FORM_LARGE, FORM_MID, FORM_SMALL, FORM_FREE, FORM_GENERAL = range(5)
 FW_KV_DENSE, FW_KV_VARLEN, FW_KV_PAGED = 0, 1, 2
 FW_DECODE_SCRATCH_BYTES = 64 << 20  # include/flywheel_hip.h
 
@@ -115,6 +116,7 @@ SIGNATURES = {
                                                _i32, _i32, _i32, _i32, _i32, _c_p]),
     "fw_prefill_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(PrefillParams)]),
     "fw_prefill": (ctypes.c_int, [ctypes.POINTER(PrefillParams), _c_p]),
+    "fw_prefill_form": (ctypes.c_int, [ctypes.POINTER(PrefillParams)]),
     "fw_rotary": (ctypes.c_int, [ctypes.POINTER(RotaryParams), _c_p]),
     "fw_clock_probe": (ctypes.c_int, [_c_p, _i32, _i32, _c_p]),
     "fw_attn_bwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnBwdParams)]),

@@ -246,6 +246,21 @@ typedef struct fw_prefill_params {
 size_t fw_prefill_workspace_bytes(const fw_prefill_params *p);
 int fw_prefill(const fw_prefill_params *p, fw_stream_t stream);
 
+/* The kernel form a call takes (nothing is launched; the forms agree to
+ * rounding): large grids, two key groups, single waves, four waves per workgroup
+ * without a key split, or the register-staged kernel for K/V rows that the
+ * copying kernels cannot address (a negative token stride or one of 2^23
+ * elements and more; at 64/64 and 192/128 also rows that do not start at
+ * multiples of 16 bytes).  Head dims without a choice return FW_FORM_LARGE. */
+enum fw_prefill_form_id {
+  FW_FORM_LARGE = 0,
+  FW_FORM_MID = 1,
+  FW_FORM_SMALL = 2,
+  FW_FORM_FREE = 3,
+  FW_FORM_GENERAL = 4
+};
+int fw_prefill_form(const fw_prefill_params *p);
+
 /*
  * Dense flash-attention backward: dq, dk, dv (bf16) from q, k, v, out, dout
  * (bf16) and the forward's lse (f32, natural log).  Replaces flash_attn_bwd

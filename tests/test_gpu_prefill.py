@@ -403,6 +403,69 @@ def test_dense_large_and_free_forms(b, h, hk, sq, sk, causal, window, softcap, s
     assert_lse(lse[-1:, hs].cpu().numpy(), rl)
 
 
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 128), (192, 128), (256, 256)])
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("step", [1 << 23, -(1 << 10), 1 << 10])
+def test_kv_token_strides(d, dv, packed, step):
+    """Token strides of K and V through the C-ABI: 16 MiB and more, and
+    negative (rows in reverse), which the register-staged kernel takes, and a
+    plain stride beside them."""
+    announce(f"kv strides d{d}/{dv} packed={packed} step {step}")
+    from flywheel_tpu import _native as N
+    rng = np.random.default_rng(76)
+    b, h, hk, sq, sk = 1, 4, 2, 45, 67
+    q, k, v = randn(rng, (b, sq, h, d)), randn(rng, (b, sk, hk, d)), randn(rng, (b, sk, hk, dv))
+    qd, out = to_dev_bf16(head_major(q)), torch.empty((b, h, sq, dv), dtype=torch.bfloat16, device=DEV)
+    buf = torch.zeros(((sk - 1) * abs(step) + 2 * hk * 256,), dtype=torch.bfloat16, device=DEV)
+    at = torch.arange(sk) * abs(step) if step > 0 else torch.arange(sk - 1, -1, -1) * -step
+    rows = buf.as_strided((buf.numel() - 4 * 256 + 1, 2 * hk * 256), (1, 1))  # [start, element]
+    for x, off in ((k, 0), (v, hk * 256)):  # K heads at 0 and 256, V heads after them
+        for i in range(hk):
+            w = x.shape[-1]
+            for t in range(sk):
+                rows[int(at[t]), off + 256 * i:off + 256 * i + w] = to_dev_bf16(x[0, t, i])
+    first = buf.data_ptr() + 2 * int(at[0])
+    cu_q = torch.tensor([0, sq], dtype=torch.int32, device=DEV)
+    cu_k = torch.tensor([0, sk], dtype=torch.int32, device=DEV)
+    p = N.PrefillParams()
+    p.kv_mode = N.FW_KV_VARLEN if packed else N.FW_KV_DENSE
+    p.q, p.out, p.k, p.v = N.ptr(qd), N.ptr(out), first, first + 2 * hk * 256
+    p.cu_seqlens_q, p.cu_seqlens_k = N.ptr(cu_q), N.ptr(cu_k)
+    p.q_stride_h, p.q_stride_t, p.o_stride_h, p.o_stride_t = sq * d, d, sq * dv, dv
+    p.k_stride_h = p.v_stride_h = 256
+    p.k_stride_t = p.v_stride_t = step
+    p.batch, p.nheads, p.nheads_k, p.head_dim, p.head_dim_v = b, h, hk, d, dv
+    p.seqlen_q, p.seqlen_k, p.max_seqlen_q = sq, sk, sq
+    p.kv_dtype, p.softmax_scale, p.causal = N.FW_BF16, d ** -0.5, 1
+    p.window_left = p.window_right = -1
+    p.k_descale = p.v_descale = 1.0
+    wide = not 0 <= step < 1 << 23
+    assert (N.lib().fw_prefill_form(p) == N.FORM_GENERAL) == wide
+    ws = torch.empty(max(1, N.lib().fw_prefill_workspace_bytes(p)), dtype=torch.uint8, device=DEV)
+    p.workspace, p.workspace_bytes = N.ptr(ws), ws.numel()
+    N.check(N.lib().fw_prefill(p, N.stream_of(qd)))
+    ro, _ = A.attention_ref(q, k, v, causal=True, round_scaled_q=True)
+    assert_close(out.float().cpu().numpy(), head_major(ro))
+
+
+@pytest.mark.parametrize("d,dv", [(64, 64), (192, 128)])
+def test_kv_rows_off_16_bytes(d, dv):
+    """Contiguous K and V that start one value into their storage."""
+    announce(f"kv off 16 bytes d{d}/{dv}")
+    rng = np.random.default_rng(77)
+    b, h, hk, sq, sk = 2, 4, 2, 70, 133
+    q, k, v = randn(rng, (b, sq, h, d)), randn(rng, (b, sk, hk, d)), randn(rng, (b, sk, hk, dv))
+
+    def shifted(x):
+        x = to_dev_bf16(head_major(x))
+        y = torch.empty(x.numel() + 1, dtype=x.dtype, device=DEV)[1:].view(x.shape)
+        return y.copy_(x)
+
+    out = flash_attn_func(to_dev_bf16(head_major(q)), shifted(k), shifted(v), causal=True)
+    ro, _ = A.attention_ref(q, k, v, causal=True, round_scaled_q=True)
+    assert_close(out.float().cpu().numpy(), head_major(ro))
+
+
 def schedule_of(qlens, klens, h, hk, causal, num_rows):
     """The (sequence, first row) pairs fw_prefill's schedule holds for packed
     sequences (head dim 128), read back from the workspace."""

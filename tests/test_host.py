@@ -163,6 +163,41 @@ def test_capi_validation_status_codes():
         assert lib.fw_rotary(r, None) == N.FW_ERR_VALUE  # no buffers
 
 
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 128), (192, 128), (256, 256)])
+def test_prefill_form_of_kv_rows(d, dv):
+    """K/V rows that a 24-bit row offset cannot reach (and, at 64/64 and
+    192/128, rows that do not start at multiples of 16 bytes) never take a
+    kernel that copies them straight into LDS; the workspace does not depend
+    on the addresses or strides."""
+    lib = N.lib()
+
+    def params(mode, kst, vst, ksh=1 << 20, k=1 << 12, v=1 << 12):
+        p = N.PrefillParams()
+        p.kv_mode, p.kv_dtype, p.k, p.v = mode, N.FW_BF16, k, v
+        p.batch, p.nheads, p.nheads_k, p.head_dim, p.head_dim_v = 2, 4, 4, d, dv
+        p.seqlen_q, p.seqlen_k, p.max_seqlen_q = 3000, 5000, 2000
+        p.k_stride_h, p.v_stride_h, p.k_stride_t, p.v_stride_t = ksh, 1 << 20, kst, vst
+        p.window_left = p.window_right = -1
+        return p
+
+    for mode in (N.FW_KV_DENSE, N.FW_KV_VARLEN):
+        plain = params(mode, d, dv)
+        assert lib.fw_prefill_form(plain) != N.FORM_GENERAL
+        for kst, vst in ((1 << 23, dv), (d, 1 << 23), (-d, dv), (d, -dv), (1 << 40, 1 << 40)):
+            p = params(mode, kst, vst)
+            assert lib.fw_prefill_form(p) == N.FORM_GENERAL, (mode, kst, vst)
+            assert lib.fw_prefill_workspace_bytes(p) == lib.fw_prefill_workspace_bytes(plain)
+        assert lib.fw_prefill_form(params(mode, (1 << 23) - 8, dv)) != N.FORM_GENERAL
+        for p in (params(mode, d + 4, dv), params(mode, d, dv, ksh=(1 << 20) + 1),
+                  params(mode, d, dv, k=(1 << 12) + 2), params(mode, d, dv, v=(1 << 12) + 8)):
+            assert (lib.fw_prefill_form(p) == N.FORM_GENERAL) == (d in (64, 192))
+    if d == 64:
+        for k, general in ((1 << 12, False), ((1 << 12) + 2, True)):
+            p = params(N.FW_KV_PAGED, 0, 0, k=k)
+            p.page_size, p.num_pages, p.max_pages = 16, 100, 50
+            assert (lib.fw_prefill_form(p) == N.FORM_GENERAL) == general
+
+
 def test_backward_workspace_planes(monkeypatch):
     """The stored backward's planes in fw_attn_bwd_workspace_bytes: bf16 P
     (and dS at 256/256) of B x H x roundup(Sq, 128) x roundup(Sk, 256), kept
