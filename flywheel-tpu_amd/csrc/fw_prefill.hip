@@ -2585,6 +2585,62 @@ static int prefill_tile_rows(const fw_prefill_params *p, int form) {
   return (form == kFormLarge && use_pingpong(p) ? kPPRows : kQT) >> pp_head_shift(p, form);
 }
 
+// Packed and paged calls at 128/128: the four-wave form, whose 128-row
+// workgroups two to a CU waste fewer rows on short sequences and even out
+// better, or the ping-pong kernel, whose 256 rows share a copied tile and
+// whose heaviest tiles split their keys.  The host knows the totals, the
+// longest query and the block table's width, not the rows' lengths.  Measured
+// (us per call, ping-pong / free, 256 CUs; sequences x length, heads):
+//   every row up to 1,024 keys long: free on any grid
+//     packed 1 x 900, 8/2 28.0 / 25.2, 4 x 100-400 20.9 / 18.3, 32 x 100-900,
+//     32/32 184.8 / 147.9; paged 1 x 200 behind 800, 8/8 31.7 / 30.4, 16 x 16-64
+//     behind 700 33.3 / 27.8, 64/8 16 x 16-64 behind 950 40.5 / 40.4 (losses only
+//     at 16/1: 64 x 5-40 behind 700 34.0 / 35.7, 64 x 16-64 behind 900 40.8 /
+//     44.2); past it one workgroup's
+//     chain sets the time of a small grid: packed 1 x 1,900, 8/2 36.3 / 39.8,
+//     paged 1 x 64 behind ~1,500 34.3 / 39.6, 4 x 20-60 35.2 / 39.6
+//   packed, from 1.75 workgroups a CU (3 x 500-1,900, 8/2, 0.8 of one: 34.6 /
+//     36.6; 4 x 1,200-1,700, 8/2, 1.4: 37.5 / 38.6; 1 x 1,900, 32/8, 1.9: 48.7 /
+//     45.7; 16 x 5-2,048, 32/8: 163 / 145) while a query row sees few keys on
+//     average: 960 with the causal mask (16 x ~1,900 538 / 526, ~2,120 721 /
+//     745), 1,280 without (32 x ~1,230, 32/8 815 / 805, 16/16 450 / 430; 4 x
+//     ~1,360 129 / 133, 8 x ~1,790 402 / 413)
+//   K and V past the 256 MB last-level cache with the causal mask, under which
+//     the order by cost runs one tile of every sequence before the next, so
+//     that every 128 rows read their keys from memory: rows of 512 keys and
+//     more stay with the ping-pong kernel (32/32, 32 x ~1,230, 614 MB: 697 / 774,
+//     64 x ~840, 838 MB 807 / 882; 64/64, 64 x ~480, 969 MB: 810 / 780; 16/16, 32
+//     x ~1,230, 307 MB: 349 / 307; not causal 32/32, 614 MB: 897 / 850)
+//   paged rows past 1,024 keys lose when all are long (32 x 200-500 behind
+//     1,400, 32/32 495 / 604, 32/8 341 / 350), except where the ping-pong
+//     workgroup holds one head and at most 128 of its 256 rows are filled
+//     (32/32, 32 x 16-64 behind 1,800 251 / 202, 16 x 81 / 71; 4 x, 0.9
+//     workgroups a CU, 45.4 / 48.9)
+static int ragged_form(const fw_prefill_params *p) {
+  const bool packed = p->kv_mode == FW_KV_VARLEN;
+  const long cus = device_cus(), batch = p->batch;
+  const long width = (long)p->max_pages * p->page_size;  // of the block table
+  const long total = packed ? p->seqlen_k : batch * width;
+  long keys = total / batch;
+  if (keys > 1920) return kFormLarge;
+  long longest = packed ? p->max_seqlen_q + std::max(0l, (long)p->seqlen_k - p->seqlen_q) : width;
+  const long grid = (long)(p->nheads >> pp_head_shift(p, kFormFree)) *
+                    max_sched_tiles(p, prefill_tile_rows(p, kFormFree));
+  const int right = p->causal ? 0 : p->window_right;
+  if (p->window_left >= 0 && right >= 0) {  // what the 128 rows of a workgroup see
+    longest = std::min(longest, (long)p->window_left + right + 128);
+    keys = std::min(keys, (long)p->window_left + right + 128);
+  }
+  const bool cached = batch * keys * p->nheads_k * 512 <= 384l << 20;
+  if (!packed && pp_head_shift(p, kFormLarge) == 0 && p->max_seqlen_q <= 128 && grid >= 2 * cus)
+    return kFormFree;
+  if (p->causal && !cached && keys >= 512) return kFormLarge;
+  if (longest <= 1024) return kFormFree;
+  if (!packed || 4 * grid < 7 * cus) return kFormLarge;
+  if (!p->causal) return keys <= 1280 ? kFormFree : kFormLarge;
+  return keys - std::min(keys, p->seqlen_q / batch) / 2 <= 960 ? kFormFree : kFormLarge;
+}
+
 // The form of a call.  Dense: by the workgroups each would launch on the CUs
 // and the key tiles T a q tile visits.  Measured (us per call, large / mid / small,
 // 256 CUs; heads x queries x keys):
@@ -2615,19 +2671,14 @@ static int prefill_tile_rows(const fw_prefill_params *p, int form) {
 //     at 1,024 (8 x 1024, not causal) 132.7 / 133.7, 8 x 2048 causal 269 / 269,
 //     2 x 2048 causal 66 / 71, 32/4 x 4096 not causal 226 / 242
 //   up to three 128-row workgroups per CU and 1,600 keys   40/8 x 2048 causal
-//     56.2 / 48.9, 32/8 x 3000 causal 76.2 / 73.8, 3 x 1024 not causal 57.6 / 51.2
-//   packed sequences, by their mean length (ragged rows even out better in
-//     smaller workgroups): 64 x ~150 91 / 65, 32 x ~500 168 / 142, 16 x ~1035
-//     244 / 230, 16 x ~1900 538 / 526, 16 x ~2120 721 / 745, 4 x ~6000 1101 / 1123
-//   paged rows, whose lengths only the device knows, by the width of the
-//     block table.
+//     56.2 / 48.9, 32/8 x 3000 causal 76.2 / 73.8, 3 x 1024 not causal 57.6 / 51.2;
+//     not where the ping-pong grid is a single round: 4 x 8/4 x 1583 not causal
+//     43.5 / 45.7, 5 x 8/8 x 1142 32.9 / 34.3
+// Varlen and paged calls at 128/128: ragged_form.
 static int form_by_size(const fw_prefill_params *p) {
   if (!(use_fr(p) || use_pingpong(p))) return kFormLarge;
-  if (p->kv_mode != FW_KV_DENSE) {
-    if (!use_pingpong(p) || p->kv_dtype != FW_BF16 || p->batch <= 0) return kFormLarge;
-    const long keys = p->kv_mode == FW_KV_VARLEN ? p->seqlen_k / p->batch : (long)p->max_pages * p->page_size;
-    return keys <= 1920 ? kFormFree : kFormLarge;
-  }
+  if (p->kv_mode != FW_KV_DENSE)
+    return use_pingpong(p) && p->kv_dtype == FW_BF16 && p->batch > 0 ? ragged_form(p) : kFormLarge;
   const long cus = device_cus();
   auto grid = [&](int form) {
     const int rows = prefill_tile_rows(p, form);
@@ -2644,7 +2695,7 @@ static int form_by_size(const fw_prefill_params *p) {
   if (mid <= 2 * cus && uneven && tiles >= 32) return kFormMid;
   if (use_pingpong(p)) {
     const long mean = p->causal ? std::min(keys, p->seqlen_k - std::min(p->seqlen_q, p->seqlen_k) / 2l) : keys;
-    if (mean < 1024 || (mid <= 3 * cus && mean < 1600)) return kFormFree;
+    if (mean < 1024 || (mid <= 3 * cus && mean < 1600 && grid(kFormLarge) > cus)) return kFormFree;
   }
   return kFormLarge;
 }

@@ -198,6 +198,52 @@ def test_prefill_form_of_kv_rows(d, dv):
             assert (lib.fw_prefill_form(p) == N.FORM_GENERAL) == general
 
 
+def ragged_params(mode, lens, h, hk, *, rows=None, width=0, causal=True, window=-1):
+    """Varlen (lens: each sequence's tokens) or paged (rows: new tokens, width:
+    the block table's keys) parameters at head dim 128."""
+    rows = rows or lens
+    p = N.PrefillParams()
+    p.kv_mode, p.kv_dtype, p.head_dim, p.nheads, p.nheads_k = mode, N.FW_BF16, 128, h, hk
+    p.batch, p.seqlen_q, p.seqlen_k = len(rows), sum(rows), sum(lens)
+    p.max_seqlen_q, p.causal = max(rows), int(causal)
+    p.window_left, p.window_right = window, -1
+    p.k_stride_t = p.v_stride_t = 128
+    p.page_size, p.max_pages, p.num_pages = 16, width // 16, 100000
+    return p
+
+
+@pytest.mark.parametrize("form,kw", [
+    # small grids with rows past 1,024 keys keep the kernel that splits keys
+    ("LARGE", dict(lens=[1900], h=8, hk=2)),
+    ("LARGE", dict(lens=[1636, 870, 500], h=8, hk=8)),
+    ("FREE", dict(lens=[900], h=8, hk=2)),
+    ("FREE", dict(lens=[1636, 870, 500], h=32, hk=8)),  # 3 workgroups a CU
+    ("FREE", dict(lens=[2048, 1000, 5, 700] * 4, h=32, hk=8)),
+    # without the causal mask a row sees twice as many keys
+    ("LARGE", dict(lens=[1800] * 8, h=32, hk=8, causal=False)),
+    ("FREE", dict(lens=[1800] * 8, h=32, hk=8)),
+    ("FREE", dict(lens=[1200] * 8, h=32, hk=8, causal=False)),
+    # K and V past the last-level cache
+    ("LARGE", dict(lens=[1230] * 32, h=32, hk=32)),
+    ("FREE", dict(lens=[1230] * 32, h=32, hk=8)),
+    ("FREE", dict(lens=[1230] * 32, h=32, hk=32, causal=False)),
+    ("FREE", dict(lens=[400] * 64, h=64, hk=64)),
+    # paged: by the block table's width
+    ("LARGE", dict(rows=[256], lens=[0], width=1600, h=8, hk=2)),
+    ("LARGE", dict(rows=[300] * 6, lens=[0], width=1680, h=8, hk=2)),
+    ("LARGE", dict(rows=[400] * 32, lens=[0], width=1920, h=32, hk=32)),
+    ("FREE", dict(rows=[256], lens=[0], width=1024, h=8, hk=2)),
+    ("FREE", dict(rows=[300] * 6, lens=[0], width=1680, h=8, hk=2, window=511)),
+    ("FREE", dict(rows=[40] * 32, lens=[0], width=1872, h=32, hk=32)),  # half of 256 rows empty
+    ("LARGE", dict(rows=[40] * 4, lens=[0], width=1872, h=32, hk=32)),
+    ("LARGE", dict(rows=[300] * 6, lens=[0], width=32768, h=8, hk=2, window=511)),
+])
+def test_ragged_prefill_form(form, kw):
+    mode = N.FW_KV_PAGED if kw.get("width") else N.FW_KV_VARLEN
+    p = ragged_params(mode, **kw)
+    assert N.lib().fw_prefill_form(p) == getattr(N, "FORM_" + form)
+
+
 def test_backward_workspace_planes(monkeypatch):
     """The stored backward's planes in fw_attn_bwd_workspace_bytes: bf16 P
     (and dS at 256/256) of B x H x roundup(Sq, 128) x roundup(Sk, 256), kept
