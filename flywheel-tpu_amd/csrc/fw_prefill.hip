@@ -1839,14 +1839,20 @@ __global__ __launch_bounds__(256, 1) void fw_prefill_d256_pair_kernel(PrefillArg
 //     runs in the loop, so 32 rows of one head finish after 1 / KG of their
 //     key tiles.
 // The groups' (m, l, O) are merged through LDS in group order at the end.
-// Measured, causal: 64/64, 4 x 32/8 heads x 1999 tokens 79.8 us, 820 TFLOP/s
-// (the register-staged kernel at two waves per SIMD: 137.7 us, 476); with
-// softcap 50 91.8 (151.6) us; 8K and 16K tokens 962 and 1,025 TFLOP/s, at which
-// the chip's power sets the clock (1.96 GHz); four waves per SIMD spill (128
-// registers): 120 us; without the exponentials 66 us, without the copies 69.
-// 192/128, 64/8 heads x 4096 tokens 288 us, 16/16 x 2048 x 3000 62 us and 52 us
-// in the mid form (register-staged: 129).  What the forms are worth on smaller
-// calls stands at prefill_form.
+// Measured, causal: 64/64, 4 x 32/8 heads x 1999 tokens 89.5 us, 731 TFLOP/s
+// (the register-staged kernel at two waves per SIMD: 137.9 us, 475); with
+// softcap 50 106.9 (152.4) us, where 8 to 10 registers spill and one is
+// reloaded on every masked tile; 32/8 heads x 8K and 16K tokens 304 and 1,143 us
+// (904 and 962 TFLOP/s); four waves per SIMD spill (128 registers).
+// 192/128, 64/8 heads x 4096 tokens 331 us, 16/16 x 2048 x 3000 73 us and 60 us
+// in the mid form (register-staged: 727 and 130).  What the forms are worth on
+// smaller calls stands at prefill_form.
+// kExactMax (64/64, 192/128): the anchor is the row's running maximum, so its
+// largest weight is exactly 1 and loses nothing when P is rounded to bf16.
+// Against 64 bits the output's error is 2.03e-3 on N(0, 1) inputs and 1.73e-3
+// with queries four times as large; with the ping-pong kernel's anchor, which
+// moves when a lane's sum passes kPsumTrigger, 2.09e-3 and 2.25e-3, in 77 us
+// at the first size above and 52 us at the last.
 constexpr int kFrKeys = 64;
 // 16-byte chunk swizzle of LDS row r: 256-byte rows as in the ping-pong kernel
 // (swz).  Rows of 128 and 384 bytes alternate between the halves of the 64
@@ -1891,6 +1897,7 @@ __global__ __launch_bounds__(64 * RW * KG, OCC) void fw_prefill_fr_kernel(Prefil
   constexpr int kRows = kFrKeys / RW;                       // key rows a wave copies
   constexpr int kNK = kRows * kKB / 1024, kNV = kRows * kVB / 1024;  // its copies per tile
   constexpr int NJ = D / 16, NC = DV / 32;
+  constexpr bool kExactMax = D != 128;  // the anchor follows the row maximum
   constexpr int kMergeB = (KG - 1) * RW * 32 * DV * 4;      // O of groups 1 .., then (m, l)
   constexpr int kLdsEnd = kMergeB + (KG - 1) * RW * 32 * 8;
   constexpr int kLds = KG * BUFS * kBuf > kLdsEnd ? KG * BUFS * kBuf : kLdsEnd;
@@ -2111,7 +2118,8 @@ __global__ __launch_bounds__(64 * RW * KG, OCC) void fw_prefill_fr_kernel(Prefil
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the K rows are read
       if (t + 1 < T) dma(t + 1, 0, kCopyK);
     }
-    // online softmax against the static anchor, as in the ping-pong kernel
+    // online softmax: against the running maximum (kExactMax), or against an
+    // anchor that a lane's sum moves, as in the ping-pong kernel
     const float m_qk = m_run == -INFINITY ? 0.f : m_run;
     if constexpr (SOFTCAP) softcap_scores<2, 16, true>(sacc, a.softcap_log2, m_qk);
     const bool full = kb >= row_lo(w_last) && kb + kFrKeys <= row_hi(w_first) && kb + kFrKeys <= sk_len;
@@ -2143,20 +2151,36 @@ __global__ __launch_bounds__(64 * RW * KG, OCC) void fw_prefill_fr_kernel(Prefil
         pop[u] = __builtin_bit_cast(bf16x8_t, pw);
       }
     };
-    exponentiate(0.f);
-    if (__any(!(psum <= kPsumTrigger) || (m_run == -INFINITY && row_has_key))) {
-      asm volatile("" ::: "memory");  // a real branch: never if-converted
-      float tmax = -INFINITY;
+    float tmax = -INFINITY;
+    auto tile_max = [&]() __attribute__((always_inline)) {
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
         for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, sacc[st][e]);
-      tmax = wave_max_xor(tmax, 32) + m_qk;
-      const float m_new = fmaxf(m_run, tmax);
+    };
+    bool rescale;
+    if constexpr (kExactMax) {
+      tile_max();
+      rescale = tmax > 0.f || (m_run == -INFINITY && tmax != -INFINITY);
+    } else {
+      exponentiate(0.f);
+      rescale = !(psum <= kPsumTrigger) || (m_run == -INFINITY && row_has_key);
+    }
+    if (__any(rescale)) {
+      asm volatile("" ::: "memory");  // a real branch: never if-converted
+      if constexpr (!kExactMax) tile_max();
+      const float m_new = fmaxf(m_run, wave_max_xor(tmax, 32) + m_qk);
       const float alpha = (m_run == -INFINITY) ? 0.f : fast_exp2(m_run - m_new);
       m_run = m_new;
       const float m_use = m_new == -INFINITY ? 0.f : m_new;
-      exponentiate(m_use - m_qk);
+      if constexpr (kExactMax) {
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) sacc[st][e] -= m_use - m_qk;
+      } else {
+        exponentiate(m_use - m_qk);
+      }
       l_run *= alpha;
 #pragma unroll
       for (int c = 0; c < NC; ++c) oacc[c] *= alpha;
@@ -2165,6 +2189,7 @@ __global__ __launch_bounds__(64 * RW * KG, OCC) void fw_prefill_fr_kernel(Prefil
         for (int e = 0; e < 16; ++e) neg_m[e] = -m_use;
       }
     }
+    if constexpr (kExactMax) exponentiate(0.f);
     l_run += psum;
     if constexpr (BUFS == 1) {  // V of tile t is in; K of tile t + 1 may be in flight
       if (t + 1 < T) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kNK) : "memory");
@@ -2649,18 +2674,18 @@ static int ragged_form(const fw_prefill_params *p) {
 //               8/2 x 1024 x 1024 26 / 18.6 / 15.1 (256 workgroups);
 //               T = 5 14.6 / 11.5 / 11.1, T = 2 11.4 / 8.9 / 9.3;
 //               two rounds of workgroups 16/4 x 1024 x 1024 26 / 19 / 23
-//     64/64     8/2 x 512 x 512 10.3 / 9.8 / 8.5, 8/2 x 64 x 4096 50 / 37 / 17
-//     192/128   8/2 x 512 x 512 15.5 / 15.2 / 12.4, 8/2 x 64 x 4096 78 / 58 / 35
+//     64/64     8/2 x 512 x 512 11.5 / 10.2 / 8.2, 8/2 x 64 x 4096 60 / 45 / 20
+//     192/128   8/2 x 512 x 512 17.2 / 16.0 / 13.0, 8/2 x 64 x 4096 94 / 69 / 48
 //   mid, while its 128-row workgroups fit the CUs, from T = 8:
 //     128/128   16/16 x 2048 x 2048 44.8 / 29.8, 16/4 x 700 x 700 21.1 / 15.7
 //               (the four-wave form below: 16.7; T = 5 14.6 / 11.5, 10.6)
-//     64/64     16/16 x 2048 x 2048 28.4 / 21.9, T = 4 8.4 / 8.3
-//     192/128   16/16 x 2048 x 3000 62.1 / 51.9, T = 8 15.6 / 15.5, T = 4 11.3 / 12.1
+//     64/64     16/16 x 2048 x 2048 33.7 / 25.7, T = 4 8.3 / 7.7
+//     192/128   16/16 x 2048 x 3000 73.3 / 59.7, T = 8 17.6 / 16.2, T = 4 12.0 / 12.3
 //   and up to two workgroups per CU when the causal mask makes long q tiles
 //   uneven (the second half of the workgroups evens them out):
 //     128/128   32/32 x 2048 x 2048 49.2 / 41.0 (not causal 58 / 66; 40 heads
 //               56 / 61), 32/8 x 1024 x 1024 twice 28.1 / 27.8
-//     64/64     32/32 x 2048 x 2048 29.3 / 26.6, 192/128 52.3 / 49.9
+//     64/64     32/32 x 2048 x 2048 33.9 / 30.5, 192/128 58.9 / 56.2
 // At 128/128 the four-wave form (two workgroups per CU, whose prologues and
 // epilogues run beside each other's loops) beats the ping-pong kernel (whose
 // 256 rows a copied tile costs less power) while a query row sees few keys on

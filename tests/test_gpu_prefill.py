@@ -8,16 +8,30 @@ import pytest
 import torch
 
 from flywheel_tpu import flash_attn_func, flash_attn_varlen_func, flash_attn_with_kvcache
+from flywheel_tpu import _native as N
 from oracle import attention as A
 from oracle import paged as P
 from tests.gpu_util import (DEV, FP8, PagedCase, announce, assert_close, assert_lse, codes_of,
                             dev_from_codes, randn, to_dev_bf16)
 
 pytestmark = pytest.mark.gpu
+FORMS = ["LARGE", "MID", "SMALL", "FREE", "GENERAL"]
 
 
 def head_major(x):  # (B, S, H, D) -> (B, H, S, D)
     return np.ascontiguousarray(x.transpose(0, 2, 1, 3))
+
+
+def dense_form(q, k, v, causal, window=(-1, -1)):
+    """The kernel form flash_attn_func takes for contiguous head-major q, k, v."""
+    p = N.PrefillParams()
+    p.kv_mode, p.kv_dtype, p.causal = N.FW_KV_DENSE, N.FW_BF16, int(causal)
+    p.k, p.v = N.ptr(k), N.ptr(v)
+    p.batch, p.nheads, p.seqlen_q, p.head_dim = q.shape
+    p.nheads_k, p.seqlen_k, p.head_dim_v = k.shape[1], k.shape[2], v.shape[3]
+    p.k_stride_t, p.v_stride_t = p.head_dim, p.head_dim_v
+    p.window_left, p.window_right = window[0], 0 if causal else window[1]
+    return FORMS[N.lib().fw_prefill_form(p)]
 
 
 @pytest.mark.parametrize(
@@ -595,6 +609,29 @@ def test_flash_attn_func_anchor_rescale(d, jump):
     ro, rl = A.attention_ref(q, k, v, round_scaled_q=True)
     assert_close(o, head_major(ro))
     assert_lse(lse.cpu().numpy(), rl)
+
+
+@pytest.mark.parametrize("d,dv", [(64, 64), (192, 128)])
+@pytest.mark.parametrize("h,s,form", [(8, 512, "SMALL"), (16, 2048, "MID"), (96, 2048, "LARGE")])
+def test_peaked_softmax_precision(d, dv, h, s, form):
+    """Queries four times N(0, 1): most of a row's weight lies on a few keys,
+    and with the row maximum as the anchor the largest weight is exactly 1.
+    The error against 64 bits is then little more than the output's rounding to
+    8 bits, 2^-7 / sqrt(12) over the root mean square of a log-uniform mantissa
+    (1.47): 1.53e-3, and 1.70e-3 to 1.73e-3 with P's rounding of the other keys
+    (emulated and measured); an anchor that lags the maximum gives 2.17e-3 and more."""
+    announce(f"peaked softmax d{d}/{dv} h{h} s{s} {form}")
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    randn = lambda *shape: torch.randn(shape, device=DEV, generator=gen)
+    q, k, v = (4 * randn(1, h, s, d)).bfloat16(), randn(1, h, s, d).bfloat16(), randn(1, h, s, dv).bfloat16()
+    assert dense_form(q, k, v, True) == form
+    out = flash_attn_func(q, k, v, causal=True)
+    qs = (q.float() * (d ** -0.5 * A.LOG2E)).bfloat16()  # the scaled queries as the kernel rounds them
+    for i in range(0, h, max(1, h // 4)):
+        w = (qs[0, i].double() @ k[0, i].double().T) / A.LOG2E
+        w = w.masked_fill(~torch.ones_like(w, dtype=torch.bool).tril(), -math.inf)
+        ref = torch.softmax(w, -1) @ v[0, i].double()
+        assert (out[0, i].double() - ref).norm() <= 1.95e-3 * ref.norm()
 
 
 @pytest.mark.parametrize("d,dv", HEAD_DIMS)
