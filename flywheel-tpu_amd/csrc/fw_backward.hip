@@ -1841,6 +1841,11 @@ extern "C" int fw_attn_bwd_d64(const fw_attn_bwd_params *p, fw_stream_t stream) 
   FW_REQUIRE(p->head_dim == 64 && head_dim_v_of(p) == 64, FW_ERR_NOT_IMPLEMENTED,
              "fw_attn_bwd_d64 takes head_dim / head_dim_v 64/64; got %d/%d", p->head_dim,
              head_dim_v_of(p));
+  FW_REQUIRE((((uintptr_t)p->q | (uintptr_t)p->k | (uintptr_t)p->v | (uintptr_t)p->dout) & 15) == 0 &&
+                 ((p->q_stride_b | p->q_stride_h | p->q_stride_t | p->k_stride_b | p->k_stride_h |
+                   p->k_stride_t | p->v_stride_b | p->v_stride_h | p->v_stride_t | p->o_stride_b |
+                   p->o_stride_h | p->o_stride_t) & 7) == 0,
+             FW_ERR_VALUE, "fw_attn_bwd_d64 copies rows of q, k, v and dout that start at multiples of 16 bytes");
   FW_REQUIRE(use_stored(p), FW_ERR_NOT_IMPLEMENTED,
              "fw_attn_bwd_d64 has no recomputing kernel for planes above the stored path's limits");
   return attn_bwd(p, (hipStream_t)stream);

@@ -8,7 +8,7 @@ feature, only when a gradient is requested.  The kernels take head dims
 64/64, 128/128, 128/256, 128/512, 256/128 and 256/256 (q and k / v and out);
 the reference's other backward pairs (64/256, 64/512, 96/96, 192/128,
 192/192, test_prefill.py:205-208,285-333), and 64/64 beyond the stored path's
-plane limits, run through them on zero-padded operands (attn_bwd_padded).  lse
+plane limits or on tensors that start off 16 bytes, run through them on zero-padded operands (attn_bwd_padded).  lse
 carries no gradient of its own.
 """
 
@@ -109,7 +109,11 @@ class FlashAttnFunction(torch.autograd.Function):
         g = dict(spec["geometry"])
         d, dv = g["head_dim"], g["head_dim_v"]
         dout, grads = torch.zeros_like(out) if dout is None else dout.contiguous(), None
-        if (d, dv) == (64, 64) or bwd_widths(d, dv) == (d, dv):
+        # the 64/64 kernels copy 16-byte pieces of rows in the forward's layout;
+        # tensors that start off 16 bytes, and other strides (saved-tensor hooks
+        # may hand those back), go through the padded copies
+        in_place = all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (q, k, v, out, dout))
+        if (d, dv) == (64, 64) and in_place or bwd_widths(d, dv) == (d, dv):
             grads = attn_bwd(q, k, v, out, dout, lse, **g)
         if grads is None:
             grads = attn_bwd_padded(q, k, v, out, dout, lse, **g)

@@ -313,7 +313,8 @@ int fw_attn_bwd(const fw_attn_bwd_params *p, fw_stream_t stream);
 /* The same at head_dim / head_dim_v 64/64, through the bf16 P plane only: the
  * size is 0 (and the call FW_ERR_NOT_IMPLEMENTED) when the plane exceeds the
  * limits above or FW_BWD_STORED=0; such calls run fw_attn_bwd on operands
- * zero-padded to 128/128. */
+ * zero-padded to 128/128.  q, k, v and dout start at multiples of 16 bytes and
+ * their strides are multiples of 8 elements (FW_ERR_VALUE otherwise). */
 size_t fw_attn_bwd_d64_workspace_bytes(const fw_attn_bwd_params *p);
 int fw_attn_bwd_d64(const fw_attn_bwd_params *p, fw_stream_t stream);
 

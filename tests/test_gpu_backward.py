@@ -362,3 +362,32 @@ def test_stored_path_matches_recompute_at_c2_shape_d256(monkeypatch):
         print(f"C2 d256 {name}: max |stored - recompute| {err:.3e}, max |grad| {scale:.3e}")
         assert torch.isfinite(a).all()
         assert err <= 1e-2 * scale, (name, err, scale)
+
+
+@pytest.mark.parametrize("shifted", ["q", "k", "v", "do", ""])
+def test_backward_d64_operands_off_16_bytes(shifted):
+    """Contiguous tensors that start one value into their storage, and (last)
+    saved tensors handed back by hooks with other strides."""
+    what = f"bwd d64 shifted {shifted or 'none, strided saved tensors'}"
+    announce(what)
+    rng = np.random.default_rng(64)
+    b, h, hk, sq, sk = 1, 4, 2, 70, 133
+    arrays = dict(q=randn(rng, (b, sq, h, 64)), k=randn(rng, (b, sk, hk, 64)),
+                  v=randn(rng, (b, sk, hk, 64)), do=randn(rng, (b, sq, h, 64)))
+
+    def put(name):
+        x = to_dev_bf16(head_major(arrays[name]))
+        if name != shifted:
+            return x
+        return torch.empty(x.numel() + 1, dtype=x.dtype, device=DEV)[1:].view(x.shape).copy_(x)
+
+    t = [put(n).requires_grad_() for n in "qkv"]
+    strided = lambda x: x.transpose(0, -1).contiguous().transpose(0, -1) if x.ndim == 4 else x
+    if shifted:
+        flash_attn_func(*t, causal=True).backward(put("do"))
+    else:
+        with torch.autograd.graph.saved_tensors_hooks(lambda x: x, strided):
+            flash_attn_func(*t, causal=True).backward(put("do"))
+    torch.cuda.synchronize()
+    check_grads([head_major(x.grad.float().cpu().numpy()) for x in t], arrays["q"], arrays["k"],
+                arrays["v"], arrays["do"], True, what)

@@ -275,6 +275,28 @@ def test_backward_workspace_planes(monkeypatch):
     assert ws(256, 256, 1, 32768) < GiB
 
 
+def test_backward_d64_operands():
+    """fw_attn_bwd_d64 copies 16-byte pieces of q, k, v and dout rows, so it
+    refuses rows that start elsewhere before any launch."""
+    def params():
+        p = N.AttnBwdParams()
+        p.batch, p.nheads, p.nheads_k, p.head_dim, p.head_dim_v = 1, 2, 2, 64, 64
+        p.seqlen_q = p.seqlen_k = 128
+        for x in ("q", "k", "v", "out", "dout", "lse", "dq", "dk", "dv"):
+            setattr(p, x, 1 << 12)
+        for x in "qkv":
+            for ax, st in (("b", 2 * 128 * 64), ("h", 128 * 64), ("t", 64)):
+                setattr(p, f"{x}_stride_{ax}", st)
+        return p
+
+    for field, value in (("q", (1 << 12) + 2), ("k", (1 << 12) + 8), ("v", (1 << 12) + 4),
+                         ("dout", (1 << 12) + 2), ("k_stride_t", 68), ("q_stride_h", 1), ("o_stride_t", 65)):
+        p = params()
+        setattr(p, field, value)
+        assert N.lib().fw_attn_bwd_d64(p, None) == N.FW_ERR_VALUE, field
+        assert b"16 bytes" in N.lib().fw_last_error(), field
+
+
 def bf(*shape):
     return torch.zeros(shape, dtype=torch.bfloat16)
 
