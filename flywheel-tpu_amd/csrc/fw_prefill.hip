@@ -2350,13 +2350,15 @@ struct SchedArgs {
 };
 // The schedule, run by one workgroup of blockDim.x threads (a power of two,
 // 64 .. 1024): a thread per tile finds its sequence by binary search over the
-// sequences' first tiles, and a counting sort over cost buckets orders the
-// tiles.  The counts are kept per run of 64 tiles, one wave each, so the order
-// (and with it the choice of split tiles) is the same on every call.  A rank
+// first tiles of the sequences with rows (no more of them than tiles), and a
+// counting sort over cost buckets orders the tiles.  The counts are kept per run
+// of 64 tiles, one wave each, so the order (and with it the choice of split
+// tiles) is the same on every call; a byte holds a run's count, which keeps the
+// tables at 37 KiB, four workgroups of fw_append_schedule_kernel on a CU.  A rank
 // sort (every tile against every other) is quadratic: 540 tiles 12,000 cycles,
 // 2,048 fifteen times that.
-constexpr int kSchedSeqs = 2048;
 constexpr int kCostBuckets = 512;
+constexpr int kSortRuns = kSortTiles / 64;
 // Costs (64-key tiles) to buckets, heaviest first: exact below 64, 32 steps
 // an octave above.
 __device__ __forceinline__ int cost_bucket(int cost) {
@@ -2368,12 +2370,13 @@ __device__ __forceinline__ int cost_bucket(int cost) {
   return kCostBuckets - 1 - c;
 }
 // Inclusive scan of v over the workgroup's threads; total = the sum of all.
-// part: 16 ints of LDS (two barriers).
-__device__ __forceinline__ int block_scan(int v, int *part, int &total) {
+// part: 16 values of LDS (two barriers).
+template <typename T>
+__device__ __forceinline__ T block_scan(T v, T *part, T &total) {
   const int tid = threadIdx.x, lane = tid & 63;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
-    const int u = __shfl_up(v, d, 64);
+    const T u = __shfl_up(v, d, 64);
     if (lane >= d) v += u;
   }
   __syncthreads();
@@ -2394,12 +2397,13 @@ __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
             cus = sa.cus;
   int32_t *sched = sa.sched, *split_code = sa.split_code;
   int *split_cnt = sa.split_cnt;
-  __shared__ int part[16];
-  __shared__ uint16_t first[kSchedSeqs];  // a sequence's first tile
-  __shared__ uint16_t seq_of[kSortTiles];
-  __shared__ uint32_t key[kSortTiles];    // bucket << 6 | rank among its run's equals
-  __shared__ __attribute__((aligned(16))) uint16_t cnt[kSortTiles / 64][kCostBuckets];
-  __shared__ int heavier[kCostBuckets];   // tiles in the buckets before
+  __shared__ long long part[16];
+  __shared__ int seqs[kSortTiles];        // the sequences with rows, and the first
+  __shared__ uint16_t first[kSortTiles];  // tile of each
+  __shared__ uint16_t seq_of[kSortTiles];  // a tile's index in them
+  __shared__ uint16_t key[kSortTiles];    // bucket << 6 | rank among its run's equals
+  __shared__ __attribute__((aligned(16))) uint8_t cnt[kCostBuckets][kSortRuns];
+  __shared__ uint16_t heavier[kCostBuckets];  // tiles in the buckets before
   const int tid = threadIdx.x, nt = blockDim.x;  // nt: a power of two, 64 .. 1024
   const int lane = tid & 63;
   {
@@ -2414,11 +2418,16 @@ __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
   const int nact = num_active ? min(max(*num_active, 0), B) : B;
   const int per = (nact + nt - 1) / nt;
   const int s0 = tid * per, s1 = min(nact, s0 + per);
-  int mine = 0;
-  for (int s = s0; s < s1; ++s) mine += (cu_q[s + 1] - cu_q[s] + qt - 1) / qt;
-  int real;
-  int idx = block_scan(mine, part, real) - mine;
-  const bool sort = real <= kSortTiles && nact <= kSchedSeqs;
+  long long mine = 0;  // tiles, and in the upper half sequences with rows
+  for (int s = s0; s < s1; ++s) {
+    const int tiles = (cu_q[s + 1] - cu_q[s] + qt - 1) / qt;
+    mine += tiles + ((long long)(tiles > 0) << 32);
+  }
+  long long sum_all;
+  const long long before_me = block_scan(mine, part, sum_all) - mine;
+  const int real = (int)sum_all, nseq = (int)((sum_all - real) >> 32);
+  int idx = (int)before_me;
+  const bool sort = real <= kSortTiles && nseq <= kSortTiles;
   const int cap = max_tiles + split_max;  // schedule slots
   int nsplit = 0;  // the nsplit heaviest tiles are split (ranks 0 .. nsplit - 1)
   if (!sort) {  // sequence order
@@ -2432,27 +2441,31 @@ __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
         }
     }
   } else {
+    int n = (int)((before_me - idx) >> 32);
     for (int s = s0; s < s1; ++s) {
-      first[s] = (uint16_t)idx;
-      idx += (cu_q[s + 1] - cu_q[s] + qt - 1) / qt;
+      const int tiles = (cu_q[s + 1] - cu_q[s] + qt - 1) / qt;
+      if (tiles <= 0) continue;
+      seqs[n] = s;
+      first[n++] = (uint16_t)idx;
+      idx += tiles;
     }
     const int runs = (real + 63) / 64;
-    for (int i = tid; i < runs * kCostBuckets / 8; i += nt)
+    for (int i = tid; i < kCostBuckets * kSortRuns / 16; i += nt)
       ((u32x4_t *)&cnt[0][0])[i] = u32x4_t{0, 0, 0, 0};
     __syncthreads();
     for (int r = tid >> 6; r < runs; r += nt >> 6) {
       const int i = 64 * r + lane;
       int lo = 0, bucket = 0;
       if (i < real) {
-        // the last sequence starting at or before tile i (sequences without
-        // rows share their successor's first tile)
-        int hi = nact;
+        // the last sequence starting at or before tile i
+        int hi = nseq;
         while (hi - lo > 1) {
           const int mid = (lo + hi) >> 1;
           if ((int)first[mid] <= i) lo = mid; else hi = mid;
         }
-        const int len = cu_q[lo + 1] - cu_q[lo];
-        const int sk = cu_k ? cu_k[lo + 1] - cu_k[lo] : seqused_k[lo] + (plus_q ? len : 0);
+        const int s = seqs[lo];
+        const int len = cu_q[s + 1] - cu_q[s];
+        const int sk = cu_k ? cu_k[s + 1] - cu_k[s] : seqused_k[s] + (plus_q ? len : 0);
         const int off = sk - len;  // bottom-right alignment, as in the kernels
         const int q0 = (i - first[lo]) * qt, last = min(q0 + qt, len) - 1;
         const int k_lo = wl >= 0 ? max(0, q0 + off - wl) : 0;
@@ -2469,29 +2482,33 @@ __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
       if (i < real) {
         const int before = __popcll(same & ((1ull << lane) - 1));
         seq_of[i] = (uint16_t)lo;
-        key[i] = (uint32_t)bucket << 6 | before;
-        if (before == 0) cnt[r][bucket] = (uint16_t)__popcll(same);
+        key[i] = (uint16_t)(bucket << 6 | before);
+        if (before == 0) cnt[bucket][r] = (uint8_t)__popcll(same);
       }
     }
     __syncthreads();
-    // cnt[r][bucket]: the bucket's tiles in earlier runs; then the buckets' sums
+    // the tiles of a bucket in runs before r (a uniform value)
+    auto in_runs = [&](int bk, int r) {
+      uint32_t sum = 0;
+#pragma unroll
+      for (int w = 0; w < kSortRuns / 4; ++w) {
+        const int bytes = min(max(r - 4 * w, 0), 4);
+        const uint32_t mask = bytes == 4 ? ~0u : (1u << (8 * bytes)) - 1;
+        sum = __builtin_amdgcn_sad_u8(((const uint32_t *)cnt[bk])[w] & mask, 0, sum);
+      }
+      return (int)sum;
+    };
     const int bpt = max(1, kCostBuckets / nt);  // buckets per thread
     int sum = 0;
     if (tid * bpt < kCostBuckets)
       for (int bk = tid * bpt; bk < (tid + 1) * bpt; ++bk) {
-        heavier[bk] = sum;
-        int run = 0;
-        for (int r = 0; r < runs; ++r) {
-          const int c = cnt[r][bk];
-          cnt[r][bk] = (uint16_t)run;
-          run += c;
-        }
-        sum += run;
+        heavier[bk] = (uint16_t)sum;
+        sum += in_runs(bk, kSortRuns);
       }
     int all;
-    const int before = block_scan(sum, part, all) - sum;
+    const int before = block_scan(sum, (int *)part, all) - sum;
     if (tid * bpt < kCostBuckets)
-      for (int bk = tid * bpt; bk < (tid + 1) * bpt; ++bk) heavier[bk] += before;
+      for (int bk = tid * bpt; bk < (tid + 1) * bpt; ++bk) heavier[bk] = (uint16_t)(heavier[bk] + before);
     __syncthreads();
     const long wgs = (long)real * ng;
     if (split_max > 0 && wgs < 16l * cus) {
@@ -2501,8 +2518,8 @@ __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
       nsplit = min(min(split_max, big), (gap + ng - 1) / ng);
     }
     for (int i = tid; i < real; i += nt) {
-      const int bucket = key[i] >> 6, s = seq_of[i], q0 = (i - first[s]) * qt;
-      const int rank = heavier[bucket] + cnt[i >> 6][bucket] + (key[i] & 63);
+      const int bucket = key[i] >> 6, n = seq_of[i], s = seqs[n], q0 = (i - first[n]) * qt;
+      const int rank = heavier[bucket] + in_runs(bucket, i >> 6) + (key[i] & 63);
       // ranks below nsplit all hold tiles of >= kMinSplitCost key tiles
       const bool split = rank < nsplit;
       if (rank < cap) {

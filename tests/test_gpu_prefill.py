@@ -480,9 +480,10 @@ def test_kv_rows_off_16_bytes(d, dv):
     assert_close(out.float().cpu().numpy(), head_major(ro))
 
 
-def schedule_of(qlens, klens, h, hk, causal, num_rows):
+def schedule_of(qlens, klens, h, hk, causal, num_rows, *, window=-1, num_active=None, codes_at=None):
     """The (sequence, first row) pairs fw_prefill's schedule holds for packed
-    sequences (head dim 128), read back from the workspace."""
+    sequences (head dim 128), read back from the workspace; with the slots' split
+    codes, held after codes_at slots, beside them."""
     from flywheel_tpu import _native as N
     dev = lambda x: torch.tensor(np.concatenate([[0], np.cumsum(x)]), dtype=torch.int32, device=DEV)
     cu_q, cu_k = dev(qlens), dev(klens)
@@ -498,13 +499,19 @@ def schedule_of(qlens, klens, h, hk, causal, num_rows):
     p.batch, p.nheads, p.nheads_k, p.head_dim = len(qlens), h, hk, 128
     p.seqlen_q, p.seqlen_k, p.max_seqlen_q = num_rows, sum(klens), max(qlens)
     p.kv_dtype, p.softmax_scale, p.causal = N.FW_BF16, 0.1, int(causal)
-    p.window_left = p.window_right = -1
+    p.window_left, p.window_right = window, -1
     p.k_descale = p.v_descale = 1.0
+    active = None if num_active is None else torch.tensor([num_active], dtype=torch.int32, device=DEV)
+    p.num_active = N.ptr(active)
     ws = torch.zeros(N.lib().fw_prefill_workspace_bytes(p), dtype=torch.uint8, device=DEV)
     p.workspace, p.workspace_bytes = N.ptr(ws), ws.numel()
     N.check(N.lib().fw_prefill(p, N.stream_of(q)))
     w = ws[:ws.numel() // 4 * 4].view(torch.int32).cpu().numpy()
-    return [(int(w[1 + 2 * i]), int(w[2 + 2 * i])) for i in range(w[0])]
+    slots = [(int(w[1 + 2 * i]), int(w[2 + 2 * i])) for i in range(w[0])]
+    if codes_at is None:
+        return slots
+    codes = -(-(1 + 2 * codes_at) * 4 // 256) * 64
+    return slots, [int(x) for x in w[codes:codes + w[0]]]
 
 
 @pytest.mark.parametrize("n,lo,hi,extra", [
@@ -526,6 +533,67 @@ def test_schedule_order(n, lo, hi, extra):
         # exact buckets below 64 key tiles, the longest here 32
         tiles.sort(key=lambda t: -min(t[1] + 32, lens[t[0]]) // 64)  # -ceil(keys / 64)
     assert got == tiles + [(-1, r) for r in range(rows, rows + extra, 32)]
+
+
+def cost_bucket(cost):
+    """The schedule's cost buckets: exact below 64 key tiles, 32 an octave above."""
+    if cost < 64:
+        return cost
+    e = cost.bit_length() - 1
+    return 64 + 32 * (e - 6) + (cost >> (e - 5)) - 32
+
+
+def tile_cost(qlen, klen, row, rows, causal, window):
+    last, off = min(row + rows, qlen) - 1, klen - qlen
+    lo = max(0, row + off - window) if window >= 0 else 0
+    hi = min(klen, last + off + 1) if causal else klen
+    return -(-hi // 64) - lo // 64 if hi > lo else 0
+
+
+def test_schedule_order_many_sequences():
+    """More than 2,048 sequences, most of them without rows: ordered as well."""
+    announce("schedule of 2600 sequences")
+    rng = np.random.default_rng(78)
+    lens = [int(x) if rng.random() < 0.3 else 0 for x in rng.integers(1, 121, 2600)]
+    tiles = [(s, r) for s in range(2600) for r in range(0, lens[s], 32)]
+    assert 1000 < len(tiles) <= 2048
+    got = schedule_of(lens, lens, 4, 1, True, sum(lens))
+    tiles.sort(key=lambda t: -tile_cost(lens[t[0]], lens[t[0]], t[1], 32, True, -1))
+    assert got == tiles
+
+
+@pytest.mark.parametrize("n,qlo,qhi,klo,khi,h,hk,causal,window,active", [
+    (40, 0, 200, 1500, 9000, 8, 1, True, -1, None),    # costs on both sides of 64 and 128
+    (40, 0, 200, 1500, 9000, 8, 1, False, -1, 33),     # sequences past num_active are padding
+    (24, 1, 400, 2000, 6000, 16, 2, True, 1500, None), # two head groups, a window
+    (3, 1, 300, 2000, 40000, 8, 1, True, -1, None),
+    (9, 100, 300, 2000, 2400, 64, 4, True, 100, None), # too few key tiles to split any
+])
+def test_schedule_split_slots(n, qlo, qhi, klo, khi, h, hk, causal, window, active):
+    """The ping-pong kernel's schedule: the heaviest tiles first, the first
+    ranks among them split in two (as many as even the last round of the CUs),
+    their second halves after every sequence tile, padding last."""
+    announce(f"schedule with splits n{n} h{h}/{hk} causal={causal} window={window} active={active}")
+    rng = np.random.default_rng(79)
+    qlens = [int(x) for x in rng.integers(qlo, qhi + 1, n)]
+    klens = [q + int(x) for q, x in zip(qlens, rng.integers(klo, khi + 1, n))]
+    rows, nact = 32, n if active is None else active  # 8 heads x 32 rows a workgroup
+    ng, total = h // 8, sum(qlens)
+    most = min(32, max(1, 256 // ng))
+    got, codes = schedule_of(qlens, klens, h, hk, causal, total, window=window, num_active=active,
+                             codes_at=-(-total // rows) + n + 1 + most)
+    cost = lambda t: tile_cost(qlens[t[0]], klens[t[0]], t[1], rows, causal, window)
+    tiles = [(s, r) for s in range(nact) for r in range(0, qlens[s], rows)]
+    tiles.sort(key=lambda t: -cost_bucket(cost(t)))
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    nsplit = 0
+    if len(tiles) * ng < 16 * cus:
+        nsplit = min(most, sum(cost(t) >= 8 for t in tiles), -(-(-len(tiles) * ng % cus) // ng))
+    assert (nsplit > 0) == (window != 100)
+    padding = [(-1, r) for r in range(sum(qlens[:nact]), total, rows)]
+    assert got == tiles + tiles[:nsplit] + padding
+    assert codes == ([2 * i for i in range(nsplit)] + [-1] * (len(tiles) - nsplit) +
+                     [2 * i + 1 for i in range(nsplit)] + [-1] * len(padding))
 
 
 @pytest.mark.parametrize("wide", [False, True])  # the four-wave form, the ping-pong kernel
