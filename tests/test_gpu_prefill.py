@@ -362,8 +362,9 @@ def test_head_dim_64_tile_edges(g, sq, sk, causal, window, softcap):
     (1, 4, 2, 600, 600, True, (-1, -1), 0.0),   # leading q tiles with fewer tiles than groups
     (1, 2, 2, 600, 520, True, (-1, -1), 0.0),   # rows that see nothing
     (2, 2, 2, 70, 900, False, (700, 3), 0.0),
+    # three key tiles: too few to split (the four-wave form at 128)
+    (1, 4, 1, 65, 130, True, (-1, -1), 0.0),
     # two key groups of four waves
-    (1, 4, 1, 65, 130, True, (-1, -1), 0.0),    # three key tiles: the second group has one
     (3, 24, 6, 129, 700, True, (-1, -1), 0.0),  # 4 heads a workgroup, 11 key tiles
     (3, 30, 15, 300, 513, False, (-1, -1), 50.0),
     # up to two such workgroups per CU
@@ -371,7 +372,7 @@ def test_head_dim_64_tile_edges(g, sq, sk, causal, window, softcap):
 ])
 def test_dense_forms(d, dv, b, h, hk, sq, sk, causal, window, softcap):
     """Dense calls whose grid leaves CUs idle: the key tiles of a q tile split
-    over waves and merged (dense_form)."""
+    over waves and merged (prefill_form)."""
     announce(f"dense form d{d}/{dv} b{b} h{h}/{hk} sq{sq} sk{sk} causal={causal} window={window}")
     rng = np.random.default_rng(72)
     q, k, v = randn(rng, (b, sq, h, d)), randn(rng, (b, sk, hk, d)), randn(rng, (b, sk, hk, dv))
@@ -389,12 +390,47 @@ def test_dense_forms(d, dv, b, h, hk, sq, sk, causal, window, softcap):
     assert_lse(lse.cpu().numpy()[:, check], rl)
 
 
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 128), (192, 128)])
+@pytest.mark.parametrize("sq,sk,causal,window", [
+    (600, 600, True, (-1, -1)),     # leading q tiles with one key tile: none for the second group
+    (600, 520, True, (-1, -1)),     # rows that see nothing: both groups' maxima -inf
+    (600, 700, False, (300, 200)),  # waves that skip their group's first tile
+    (600, 700, True, (480, -1)),
+])
+def test_two_key_groups(d, dv, sq, sk, causal, window):
+    announce(f"two key groups d{d}/{dv} sq{sq} sk{sk} causal={causal} window={window}")
+    rng = np.random.default_rng(80)
+    h = 16  # 304 workgroups of 32 rows, 80 of 128
+    q, k, v = randn(rng, (1, sq, h, d)), randn(rng, (1, sk, h, d)), randn(rng, (1, sk, h, dv))
+    qt, kt, vt = (to_dev_bf16(head_major(x)) for x in (q, k, v))
+    assert dense_form(qt, kt, vt, causal, window) == "MID"
+    out, lse = flash_attn_func(qt, kt, vt, causal=causal, window_size=window, return_softmax_lse=True)
+    ro, rl = A.attention_ref(q, k, v, causal=causal, window_size=window, round_scaled_q=True)
+    assert_close(out.float().cpu().numpy(), head_major(ro))
+    assert_lse(lse.cpu().numpy(), rl)
+
+
+# One call per kernel form: (d, dv, h, sq, sk, form)
+FORM_CALLS = [
+    (64, 64, 4, 256, 768, "SMALL"), (64, 64, 60, 256, 768, "MID"), (64, 64, 132, 256, 768, "LARGE"),
+    (128, 128, 4, 256, 768, "SMALL"), (128, 128, 60, 256, 768, "MID"),
+    (128, 128, 132, 256, 768, "FREE"), (128, 128, 132, 256, 1728, "LARGE"),
+    (128, 128, 256, 512, 1728, "LARGE"),  # pairs of q tiles
+    (192, 128, 4, 256, 768, "SMALL"), (192, 128, 60, 256, 768, "MID"),
+    (192, 128, 132, 256, 768, "LARGE"),
+    (256, 256, 256, 256, 768, "LARGE"),  # pairs of q tiles
+]
+
+
 @pytest.mark.parametrize("b,h,hk,sq,sk,causal,window,softcap,sinks", [
     # the ping-pong kernel (many rows, at least 1,600 keys a row): ragged ends
     # on both sides, 1, 2 and 8 heads a workgroup
     (1, 30, 30, 1150, 2305, False, (-1, -1), 0.0, True),
     (2, 18, 9, 1055, 2113, False, (1800, 700), 50.0, False),
     (1, 64, 8, 2309, 3457, True, (-1, -1), 0.0, False),
+    # softcap tanh: exact, and the degree-5 polynomial
+    (1, 64, 8, 1055, 2113, False, (-1, -1), 5.0, False),
+    (1, 64, 8, 1055, 2113, False, (-1, -1), 20.0, False),
     # the four-wave form: tile edges, 1, 2 and 4 heads a workgroup
     (5, 24, 8, 257, 257, True, (-1, -1), 0.0, True),
     (9, 10, 5, 129, 191, False, (64, 17), 30.0, False),
@@ -677,6 +713,41 @@ def test_flash_attn_func_anchor_rescale(d, jump):
     ro, rl = A.attention_ref(q, k, v, round_scaled_q=True)
     assert_close(o, head_major(ro))
     assert_lse(lse.cpu().numpy(), rl)
+
+
+@pytest.mark.parametrize("d,dv,h,sq,sk,form", FORM_CALLS)
+@pytest.mark.parametrize("jump", [40.0, 600.0])
+def test_anchor_rescale_forms(d, dv, h, sq, sk, form, jump):
+    """The rescale of test_flash_attn_func_anchor_rescale in every form of the
+    prefill kernels: scores 0, J/2 and J and values 1, 2 and 3 by thirds of the
+    keys, out ~3 and lse = J ln 2 + ln(sk / 3) in closed form."""
+    announce(f"anchor rescale d{d}/{dv} h{h} sq{sq} sk{sk} {form} jump {jump}")
+    y = jump / (math.sqrt(d) * A.LOG2E)
+    third = torch.arange(sk, device=DEV) // (sk // 3)
+    rows = lambda w, x: x.to(torch.bfloat16).reshape(1, 1, sk, 1).expand(1, 1, sk, w).contiguous()
+    q = torch.ones((1, h, sq, d), dtype=torch.bfloat16, device=DEV)
+    k, v = rows(d, third * (y / 2)), rows(dv, third + 1)
+    assert dense_form(q, k, v, False) == form
+    out, lse = flash_attn_func(q, k, v, return_softmax_lse=True)
+    # the last third's score with q scaled and rounded, and k, as bf16 (2^-8 each)
+    qs = torch.tensor(d ** -0.5 * A.LOG2E).to(torch.bfloat16).double()
+    score = float(qs * k[0, 0, -1, 0].double().cpu()) * d / A.LOG2E
+    assert (out.float() - 3.0).abs().max() <= 2e-2
+    assert (lse - (score + math.log(sk // 3))).abs().max() <= 1e-3
+
+
+@pytest.mark.parametrize("d,dv,h,sq,sk,form", FORM_CALLS)
+def test_bitwise_repeat_forms(d, dv, h, sq, sk, form):
+    """Repeats are bitwise equal in every form (a race on the shared LDS
+    buffers would show as a difference)."""
+    announce(f"repeat d{d}/{dv} h{h} sq{sq} sk{sk} {form}")
+    gen = torch.Generator(device=DEV).manual_seed(81)
+    q, k, v = (torch.randn(x, generator=gen, device=DEV, dtype=torch.bfloat16)
+               for x in ((1, h, sq, d), (1, h // 2, sk, d), (1, h // 2, sk, dv)))
+    assert dense_form(q, k, v, False) == form
+    ref = flash_attn_func(q, k, v)
+    for _ in range(20):
+        assert torch.equal(flash_attn_func(q, k, v), ref)
 
 
 @pytest.mark.parametrize("d,dv", [(64, 64), (192, 128)])

@@ -155,7 +155,8 @@ def test_random_case(kind, seed):
 @pytest.mark.parametrize("seed", range(8))
 @pytest.mark.parametrize("d", [64, 256])
 def test_random_case_head_dims(d, kind, seed):
-    """The same draws at head_dim 64 (register-staged prefill kernel, decode)
+    """The same draws at head_dim 64 (the free-running prefill kernel, the
+    register-staged one over fp8 pools, decode)
     and 256 (the head_dim-256 prefill kernel over bf16 and fp8 pools, decode)."""
     one_case(5000 + 100 * d + 1000 * kind + seed, kind, d)
 

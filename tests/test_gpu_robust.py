@@ -139,7 +139,9 @@ def test_verify_window_and_chunked_prefill_ignore_nan(dtype, hd):
 @pytest.mark.parametrize("hd", [128, 256])
 @pytest.mark.parametrize("dtype", ["bf16", "e4m3"])
 @pytest.mark.parametrize("bad_id", [-1, 1 << 30])
-def test_invalid_page_ids_read_as_zero_rows(dtype, bad_id, hd):
+@pytest.mark.parametrize("max_pages", [None, 130])  # 1,504 and 2,080 keys: the bf16
+# prefill at 128 runs the four-wave form and the ping-pong kernel
+def test_invalid_page_ids_read_as_zero_rows(dtype, bad_id, hd, max_pages):
     """Decode (with the fused append), the folded verify window and the paged
     varlen prefill over a table with out-of-range entries: nothing is read or
     written through them, and their keys act as zero K and V rows.  Expected:
@@ -150,7 +152,7 @@ def test_invalid_page_ids_read_as_zero_rows(dtype, bad_id, hd):
     dt = torch.bfloat16 if dtype == "bf16" else FP8[dtype]
     lengths = [64, 700, 333, 1500]
     case = PagedCase(rng, batch=4, nheads=8, nheads_k=2, lengths=lengths, new_tokens=[1] * 4,
-                     head_dim=hd, dtype=dt, extra_pages=2)
+                     head_dim=hd, dtype=dt, extra_pages=2, max_pages=max_pages)
     poison_unused_slots(case, case.lengths)
     bad = {0: [1], 1: [0, 5, 6, 30], 2: [19], 3: [92]}  # full pages before each row's append page
     table = case.table.copy()
