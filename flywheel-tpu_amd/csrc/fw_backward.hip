@@ -610,7 +610,8 @@ __device__ __forceinline__ int row_swz(int r) {
 
 template <bool CAUSAL, int D>
 __global__ __launch_bounds__(256, D == 64 ? 3 : D == 128 ? 2 : 1) void fw_bwd_dq_store_kernel(BwdArgs a) {
-  // D = 64, 128 or 256 (q, k, v and out).  At 256 the kernel also stores dS
+  // D = 64, 128 or 256 (q, k, v and out).  At 64 three workgroups share a CU at
+  // 168 registers (the causal form spills 2 before its loop).  At 256 the kernel also stores dS
   // beside P, and runs one wave per SIMD (q, dout and dq of 32 rows take 256
   // registers).
   constexpr int kRow = 2 * D;          // bytes of one K / V row
@@ -690,7 +691,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : D == 128 ? 2 : 1) void fw_bwd_dq
 
   // ---- copies: wave w moves key rows 16w .. 16w + 15 of K and of V (kRPI
   // rows per instruction; lane: row kRPI i + lane / kLPR, LDS slot lane % kLPR
-  // holding global chunk slot ^ kv_swz(row))
+  // holding global chunk slot ^ row_swz<D>(row))
   constexpr int kRPI = 1024 / kRow, kLPR = 64 / kRPI;
   const uint32_t wu = __builtin_amdgcn_readfirstlane(w);
   const uint8_t *kg = sgpr_ptr((const uint8_t *)(a.k + (size_t)b * a.ksb + (size_t)hk * a.ksh));
@@ -1765,10 +1766,16 @@ bool use_stored(const fw_attn_bwd_params *p) {
          stored_planes(p) * stored_plane_bytes(p) <= kStoredMaxBytes;
 }
 
-// The stored dk / dv kernel at 128/128 runs two workgroups per CU and wants
-// about four per CU so that the causal imbalance evens out; the recomputing
-// one runs one.  At 256/256 (128-key workgroups, one per CU) the split is
-// chosen over its own grid.
+// The stored dk / dv kernels run one workgroup of 256 keys per CU at 128/128
+// and three of 128 keys at 64/64; pick_split counts 128-key blocks, of which
+// 1,024 (two rounds of workgroups at 128, one and a third at 64) even out the
+// causal imbalance.  Backward in us, causal, at targets 512 / 768 / 1,024 / 1,536:
+//   64/64    1 x 32/4 x 4096 417 / 331 / 328 / 329, 4 x 32/8 x 2000 422 / 339 / 331 /
+//            360, 2 x 64/8 x 2048 435 / 343 / 342 / 365
+//   128/128  620 / 545 / 541 / 538, 641 / 590 / 582 / 634, 672 / 601 / 597 / 642
+//            (8 x 32/8 x 512 141 / 157 / 158 / 158)
+// The recomputing kernel runs one per CU.  At 256/256 (128-key workgroups, one
+// per CU) the split is chosen over its own grid.
 int bwd_split(const fw_attn_bwd_params *p) {
   if (use_stored(p) && p->head_dim == 256) {
     const int G = p->nheads / p->nheads_k;
