@@ -2419,8 +2419,10 @@ __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
   const int per = (nact + nt - 1) / nt;
   const int s0 = tid * per, s1 = min(nact, s0 + per);
   long long mine = 0;  // tiles, and in the upper half sequences with rows
+  int tiles0 = 0;      // of sequence s0: the only one in batches up to nt
   for (int s = s0; s < s1; ++s) {
     const int tiles = (cu_q[s + 1] - cu_q[s] + qt - 1) / qt;
+    if (s == s0) tiles0 = tiles;
     mine += tiles + ((long long)(tiles > 0) << 32);
   }
   long long sum_all;
@@ -2443,7 +2445,7 @@ __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
   } else {
     int n = (int)((before_me - idx) >> 32);
     for (int s = s0; s < s1; ++s) {
-      const int tiles = (cu_q[s + 1] - cu_q[s] + qt - 1) / qt;
+      const int tiles = s == s0 ? tiles0 : (cu_q[s + 1] - cu_q[s] + qt - 1) / qt;
       if (tiles <= 0) continue;
       seqs[n] = s;
       first[n++] = (uint16_t)idx;
