@@ -873,9 +873,9 @@ __device__ __forceinline__ bf16x8_t tr_rm(uint32_t Rb, int col, int u, int lane)
 // At head dim 64 a workgroup is 4 waves = 128 keys and three share a CU: both
 // stored kernels then run three waves per SIMD, and the plane (half as much
 // matrix work per P byte as at 128) is streamed by more waves.  4 x 16/16
-// heads x 2000 tokens, causal: dq 88 us and dk / dv 95 us, where the 128
+// heads x 2000 tokens, causal: dq 86 us and dk / dv 93 us, where the 128
 // kernels on zero-padded operands took 123 and 140 beside 95 us of padding
-// and slicing (forward + backward 412 -> 235 us).
+// and slicing (forward + backward 418 -> 241 us).
 constexpr int kSQ = 32;                    // query rows per item
 // waves (32 keys each) per workgroup: 8, one workgroup per CU, at head dim
 // 128; 4, three per CU (161 registers), at 64

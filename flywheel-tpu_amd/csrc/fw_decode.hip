@@ -889,7 +889,7 @@ static int decode_launch(const fw_decode_params *p, void *ws, size_t ws_bytes,
   // nw segments: 32,000 keys beside 63 rows of 60, 73 -> 53 us; four groups at
   // 16 rows, 1,024 threads for rows of three segments, cost a batch of 128 fp8
   // verify windows 1%).  One row of 4,001 keys, 32/8 heads, has 126 segments:
-  // one group merged them in 23 us of dependent loads, 16 groups in 6.
+  // one group merged them in 23 us of dependent loads, 16 groups in 9.
   auto merge = [&](auto dc) {
     constexpr int D = decltype(dc)::value;
     c.groups = 1;
