@@ -1845,8 +1845,9 @@ __global__ __launch_bounds__(256, 1) void fw_prefill_d256_pair_kernel(PrefillArg
 // reloaded on every masked tile; 32/8 heads x 8K and 16K tokens 304 and 1,143 us
 // (904 and 962 TFLOP/s); four waves per SIMD spill (128 registers).
 // 192/128, 64/8 heads x 4096 tokens 331 us, 16/16 x 2048 x 3000 73 us and 60 us
-// in the mid form (register-staged: 727 and 130).  What the forms are worth on
-// smaller calls stands at prefill_form.
+// in the mid form (register-staged: 727 and 130); its softcap forms spill three
+// registers, outside the loop.  What the forms are worth on smaller calls stands
+// at prefill_form.
 // kExactMax (64/64, 192/128): the anchor is the row's running maximum, so its
 // largest weight is exactly 1 and loses nothing when P is rounded to bf16.
 // Against 64 bits the output's error is 2.03e-3 on N(0, 1) inputs and 1.73e-3
