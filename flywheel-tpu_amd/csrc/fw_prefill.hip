@@ -2355,9 +2355,11 @@ struct SchedArgs {
 // counting sort over cost buckets orders the tiles.  The counts are kept per run
 // of 64 tiles, one wave each, so the order (and with it the choice of split
 // tiles) is the same on every call; a byte holds a run's count, which keeps the
-// tables at 37 KiB, four workgroups of fw_append_schedule_kernel on a CU.  A rank
-// sort (every tile against every other) is quadratic: 540 tiles 12,000 cycles,
-// 2,048 fifteen times that.
+// tables at 37 KiB, four workgroups of fw_append_schedule_kernel on a CU.  Up to
+// 64 tiles are ranked by ballots within a wave instead, without the tables (three
+// packed sequences of up to 26 rows, 2/2 heads at 64: the call 10.1 -> 8.5 us).
+// A rank sort (every tile against every other) is quadratic: 540 tiles 12,000
+// cycles, 2,048 fifteen times that.
 constexpr int kCostBuckets = 512;
 constexpr int kSortRuns = kSortTiles / 64;
 // Costs (64-key tiles) to buckets, heaviest first: exact below 64, 32 steps
@@ -2453,76 +2455,19 @@ __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
       idx += tiles;
     }
     const int runs = (real + 63) / 64;
-    for (int i = tid; i < kCostBuckets * kSortRuns / 16; i += nt)
-      ((u32x4_t *)&cnt[0][0])[i] = u32x4_t{0, 0, 0, 0};
-    __syncthreads();
-    for (int r = tid >> 6; r < runs; r += nt >> 6) {
-      const int i = 64 * r + lane;
-      int lo = 0, bucket = 0;
-      if (i < real) {
-        // the last sequence starting at or before tile i
-        int hi = nseq;
-        while (hi - lo > 1) {
-          const int mid = (lo + hi) >> 1;
-          if ((int)first[mid] <= i) lo = mid; else hi = mid;
-        }
-        const int s = seqs[lo];
-        const int len = cu_q[s + 1] - cu_q[s];
-        const int sk = cu_k ? cu_k[s + 1] - cu_k[s] : seqused_k[s] + (plus_q ? len : 0);
-        const int off = sk - len;  // bottom-right alignment, as in the kernels
-        const int q0 = (i - first[lo]) * qt, last = min(q0 + qt, len) - 1;
-        const int k_lo = wl >= 0 ? max(0, q0 + off - wl) : 0;
-        const int k_hi = wr >= 0 ? min(sk, last + off + wr + 1) : sk;
-        bucket = cost_bucket(k_hi > k_lo ? (k_hi + kKT - 1) / kKT - k_lo / kKT : 0);
-      }
-      // the run's tiles of the same bucket, one bit each
-      uint64_t same = __ballot(i < real);
-#pragma unroll
-      for (int bit = 0; bit < 9; ++bit) {
-        const uint64_t set = __ballot((bucket >> bit) & 1);
-        same &= (bucket >> bit) & 1 ? set : ~set;
-      }
-      if (i < real) {
-        const int before = __popcll(same & ((1ull << lane) - 1));
-        seq_of[i] = (uint16_t)lo;
-        key[i] = (uint16_t)(bucket << 6 | before);
-        if (before == 0) cnt[bucket][r] = (uint8_t)__popcll(same);
-      }
-    }
-    __syncthreads();
-    // the tiles of a bucket in runs before r (a uniform value)
-    auto in_runs = [&](int bk, int r) {
-      uint32_t sum = 0;
-#pragma unroll
-      for (int w = 0; w < kSortRuns / 4; ++w) {
-        const int bytes = min(max(r - 4 * w, 0), 4);
-        const uint32_t mask = bytes == 4 ? ~0u : (1u << (8 * bytes)) - 1;
-        sum = __builtin_amdgcn_sad_u8(((const uint32_t *)cnt[bk])[w] & mask, 0, sum);
-      }
-      return (int)sum;
-    };
-    const int bpt = max(1, kCostBuckets / nt);  // buckets per thread
-    int sum = 0;
-    if (tid * bpt < kCostBuckets)
-      for (int bk = tid * bpt; bk < (tid + 1) * bpt; ++bk) {
-        heavier[bk] = (uint16_t)sum;
-        sum += in_runs(bk, kSortRuns);
-      }
-    int all;
-    const int before = block_scan(sum, (int *)part, all) - sum;
-    if (tid * bpt < kCostBuckets)
-      for (int bk = tid * bpt; bk < (tid + 1) * bpt; ++bk) heavier[bk] = (uint16_t)(heavier[bk] + before);
+    const bool one_run = runs == 1;  // ranked within a wave: every wave does it, wave 0 writes
+    if (!one_run)
+      for (int i = tid; i < kCostBuckets * kSortRuns / 16; i += nt)
+        ((u32x4_t *)&cnt[0][0])[i] = u32x4_t{0, 0, 0, 0};
     __syncthreads();
     const long wgs = (long)real * ng;
-    if (split_max > 0 && wgs < 16l * cus) {
+    // big: tiles of at least kMinSplitCost key tiles
+    auto splits = [&](int big) {
+      if (split_max == 0 || wgs >= 16l * cus) return 0;
       const int gap = (int)((cus - wgs % cus) % cus);
-      // tiles of at least kMinSplitCost key tiles
-      const int big = heavier[cost_bucket(kMinSplitCost - 1)];
-      nsplit = min(min(split_max, big), (gap + ng - 1) / ng);
-    }
-    for (int i = tid; i < real; i += nt) {
-      const int bucket = key[i] >> 6, n = seq_of[i], s = seqs[n], q0 = (i - first[n]) * qt;
-      const int rank = heavier[bucket] + in_runs(bucket, i >> 6) + (key[i] & 63);
+      return min(min(split_max, big), (gap + ng - 1) / ng);
+    };
+    auto place = [&](int s, int q0, int rank) {
       // ranks below nsplit all hold tiles of >= kMinSplitCost key tiles
       const bool split = rank < nsplit;
       if (rank < cap) {
@@ -2535,6 +2480,78 @@ __device__ __forceinline__ void schedule_body(const SchedArgs &sa) {
         sched[1 + 2 * r2] = s;
         sched[2 + 2 * r2] = q0;
         split_code[r2] = 2 * rank + 1;
+      }
+    };
+    for (int r = one_run ? 0 : tid >> 6; r < runs; r += nt >> 6) {
+      const int i = 64 * r + lane;
+      int lo = 0, bucket = 0, q0 = 0, s = 0;
+      if (i < real) {
+        // the last sequence starting at or before tile i
+        int hi = nseq;
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if ((int)first[mid] <= i) lo = mid; else hi = mid;
+        }
+        s = seqs[lo];
+        const int len = cu_q[s + 1] - cu_q[s];
+        const int sk = cu_k ? cu_k[s + 1] - cu_k[s] : seqused_k[s] + (plus_q ? len : 0);
+        const int off = sk - len;  // bottom-right alignment, as in the kernels
+        q0 = (i - first[lo]) * qt;
+        const int last = min(q0 + qt, len) - 1;
+        const int k_lo = wl >= 0 ? max(0, q0 + off - wl) : 0;
+        const int k_hi = wr >= 0 ? min(sk, last + off + wr + 1) : sk;
+        bucket = cost_bucket(k_hi > k_lo ? (k_hi + kKT - 1) / kKT - k_lo / kKT : 0);
+      }
+      // the run's tiles of the same bucket, one bit each, and how many are heavier
+      uint64_t same = __ballot(i < real);
+      int above = 0;
+#pragma unroll
+      for (int bit = 8; bit >= 0; --bit) {
+        const uint64_t set = __ballot((bucket >> bit) & 1);
+        if ((bucket >> bit) & 1) above += __popcll(same & ~set);
+        same &= (bucket >> bit) & 1 ? set : ~set;
+      }
+      const int before = __popcll(same & ((1ull << lane) - 1));
+      if (one_run) {
+        nsplit = splits(__popcll(__ballot(i < real && bucket < cost_bucket(kMinSplitCost - 1))));
+        if (tid < real) place(s, q0, above + before);
+        break;
+      }
+      if (i < real) {
+        seq_of[i] = (uint16_t)lo;
+        key[i] = (uint16_t)(bucket << 6 | before);
+        if (before == 0) cnt[bucket][r] = (uint8_t)__popcll(same);
+      }
+    }
+    if (!one_run) {
+      __syncthreads();
+      // the tiles of a bucket in runs before r (a uniform value)
+      auto in_runs = [&](int bk, int r) {
+        uint32_t sum = 0;
+#pragma unroll
+        for (int w = 0; w < kSortRuns / 4; ++w) {
+          const int bytes = min(max(r - 4 * w, 0), 4);
+          const uint32_t mask = bytes == 4 ? ~0u : (1u << (8 * bytes)) - 1;
+          sum = __builtin_amdgcn_sad_u8(((const uint32_t *)cnt[bk])[w] & mask, 0, sum);
+        }
+        return (int)sum;
+      };
+      const int bpt = max(1, kCostBuckets / nt);  // buckets per thread
+      int sum = 0;
+      if (tid * bpt < kCostBuckets)
+        for (int bk = tid * bpt; bk < (tid + 1) * bpt; ++bk) {
+          heavier[bk] = (uint16_t)sum;
+          sum += in_runs(bk, kSortRuns);
+        }
+      int all;
+      const int before = block_scan(sum, (int *)part, all) - sum;
+      if (tid * bpt < kCostBuckets)
+        for (int bk = tid * bpt; bk < (tid + 1) * bpt; ++bk) heavier[bk] = (uint16_t)(heavier[bk] + before);
+      __syncthreads();
+      nsplit = splits(heavier[cost_bucket(kMinSplitCost - 1)]);
+      for (int i = tid; i < real; i += nt) {
+        const int bucket = key[i] >> 6, n = seq_of[i];
+        place(seqs[n], (i - first[n]) * qt, heavier[bucket] + in_runs(bucket, i >> 6) + (key[i] & 63));
       }
     }
   }
