@@ -2660,7 +2660,13 @@ static int prefill_tile_rows(const fw_prefill_params *p, int form) {
 //     at 16/1: 64 x 5-40 behind 700 34.0 / 35.7, 64 x 16-64 behind 900 40.8 /
 //     44.2); past it one workgroup's
 //     chain sets the time of a small grid: packed 1 x 1,900, 8/2 36.3 / 39.8,
-//     paged 1 x 64 behind ~1,500 34.3 / 39.6, 4 x 20-60 35.2 / 39.6
+//     paged 1 x 64 behind ~1,500 34.3 / 39.6, 4 x 20-60 35.2 / 39.6; on a larger
+//     grid where one row is much longer than the rest (packed 32 x ~350, one behind
+//     6,000, 4/4, 1.9 workgroups a CU: 77.5 / 113.0; 32 x ~165 at 16/2, 3.1 of them:
+//     86 / 106; 8 x ~460 at 32/8, 3.9: 124 / 119; 32 x ~340 at 32/4, 11.8: 162 / 121)
+//   with max_seqlen_k; without it a packed call's longest row is bounded by its
+//     queries and all keys beyond the total of queries (3 x up to 8 rows behind
+//     500 keys each, 6/2: 21.6 / 17.8)
 //   packed, from 1.75 workgroups a CU (3 x 500-1,900, 8/2, 0.8 of one: 34.6 /
 //     36.6; 4 x 1,200-1,700, 8/2, 1.4: 37.5 / 38.6; 1 x 1,900, 32/8, 1.9: 48.7 /
 //     45.7; 16 x 5-2,048, 32/8: 163 / 145) while a query row sees few keys on
@@ -2686,6 +2692,7 @@ static int ragged_form(const fw_prefill_params *p) {
   long keys = total / batch;
   if (keys > 1920) return kFormLarge;
   long longest = packed ? p->max_seqlen_q + std::max(0l, (long)p->seqlen_k - p->seqlen_q) : width;
+  if (packed && p->max_seqlen_k > 0) longest = std::min(longest, (long)p->max_seqlen_k);
   const long grid = (long)(p->nheads >> pp_head_shift(p, kFormFree)) *
                     max_sched_tiles(p, prefill_tile_rows(p, kFormFree));
   const int right = p->causal ? 0 : p->window_right;
@@ -2698,7 +2705,7 @@ static int ragged_form(const fw_prefill_params *p) {
     return kFormFree;
   if (p->causal && !cached && keys >= 512) return kFormLarge;
   if (longest <= 1024) return kFormFree;
-  if (!packed || 4 * grid < 7 * cus) return kFormLarge;
+  if (!packed || 4 * grid < 7 * cus || (longest > 4096 && 2 * grid < 7 * cus)) return kFormLarge;
   if (!p->causal) return keys <= 1280 ? kFormFree : kFormLarge;
   return keys - std::min(keys, p->seqlen_q / batch) / 2 <= 960 ? kFormFree : kFormLarge;
 }

@@ -69,7 +69,7 @@ class PrefillParams(ctypes.Structure):
         ("rotary_rows", _i32), ("rotary_f32", _i32), ("rotary_interleaved", _i32),
         ("seqused_k_excludes_q", _i32),
         ("k_descale_ptr", _c_p), ("v_descale_ptr", _c_p),
-        ("head_dim_v", _i32),
+        ("head_dim_v", _i32), ("max_seqlen_k", _i32),
         ("k_new", _c_p), ("v_new", _c_p),
     ]
 

@@ -47,7 +47,8 @@ def _split_token_major(x, head_dim):
 
 def _run_prefill(mode, q, k, v, out, lse, *, qs, ks, vs, os_, ls, batch, nheads, nheads_k,
                  head_dim, seqlen_q, seqlen_k, causal, window_size, softmax_scale, softcap,
-                 sinks, cu_q=None, cu_k=None, max_seqlen_q=0, q_rotary=None, head_dim_v=0):
+                 sinks, cu_q=None, cu_k=None, max_seqlen_q=0, max_seqlen_k=0, q_rotary=None,
+                 head_dim_v=0):
     left, right = effective_window(causal, window_size)
     ptr = N.ptr
     p = N.PrefillParams(  # in field order: one call, not an attribute at a time
@@ -55,7 +56,7 @@ def _run_prefill(mode, q, k, v, out, lse, *, qs, ks, vs, os_, ls, batch, nheads,
         ptr(sinks), None, 0, *qs, *os_, *ks, *vs, *ls, batch, nheads, nheads_k, head_dim,
         seqlen_q, seqlen_k, max_seqlen_q, 0, 0, 0, N.FW_BF16, softmax_scale, float(softcap),
         int(causal), left, right, 1.0, 1.0)
-    p.head_dim_v = head_dim_v
+    p.head_dim_v, p.max_seqlen_k = head_dim_v, max_seqlen_k
     keep = None if q_rotary is None else R.set_q_rotary(p, *q_rotary, q.device)
     lib = N.lib()
     nbytes = 0 if mode == N.FW_KV_DENSE else lib.fw_prefill_workspace_bytes(p)
@@ -505,7 +506,7 @@ def flash_attn_varlen_func(
                      seqlen_q=total_q, seqlen_k=total_k, causal=causal,
                      window_size=window_size, softmax_scale=resolve_scale(softmax_scale, d),
                      softcap=softcap, sinks=sinks, cu_q=cu_q_dev, cu_k=cu_k_dev,
-                     max_seqlen_q=int(max_seqlen_q),
+                     max_seqlen_q=int(max_seqlen_q), max_seqlen_k=int(max_seqlen_k),
                      q_rotary=None if tables is None else (tables, rotary_interleaved),
                      head_dim_v=dv)
         return out, lse
@@ -577,7 +578,7 @@ def _flash_attn_func_pcp_causal_offset(
                  ls=(0, q_len), batch=1, nheads=nheads, nheads_k=nkv, head_dim=d,
                  seqlen_q=q_len, seqlen_k=kv_len, causal=True, window_size=(-1, -1),
                  softmax_scale=resolve_scale(softmax_scale, d), softcap=0.0, sinks=None,
-                 cu_q=cu_q, cu_k=cu_k, max_seqlen_q=q_len)
+                 cu_q=cu_q, cu_k=cu_k, max_seqlen_q=q_len, max_seqlen_k=kv_len)
     out = out.reshape(q.shape)
     if return_softmax_lse:
         return out, lse.reshape(1, nheads, q_len)  # (batch, nheads, q_len) either way

@@ -232,6 +232,9 @@ typedef struct fw_prefill_params {
    * 256/128); a paged pool has one head dim of 64,
    * 128 or 256; the fused RoPE takes head_dim_v == head_dim. */
   int32_t head_dim_v;
+  /* Varlen, optional: the longest sequence's keys, 0 = not known.  Only the
+   * choice of the kernel form reads it. */
+  int32_t max_seqlen_k;
   /* Paged only, optional: new K and V rows (seqlen_q, nheads_k, head_dim) in
    * the pool's dtype, appended before the attention in the same launch as the
    * schedule: row i of request r (cu_seqlens_q[r] <= i < cu_seqlens_q[r + 1],

@@ -198,7 +198,8 @@ def test_prefill_form_of_kv_rows(d, dv):
             assert (lib.fw_prefill_form(p) == N.FORM_GENERAL) == general
 
 
-def ragged_params(mode, lens, h, hk, *, rows=None, width=0, causal=True, window=-1):
+def ragged_params(mode, lens, h, hk, *, rows=None, width=0, causal=True, window=-1,
+                  longest=0):
     """Varlen (lens: each sequence's tokens) or paged (rows: new tokens, width:
     the block table's keys) parameters at head dim 128."""
     rows = rows or lens
@@ -206,7 +207,7 @@ def ragged_params(mode, lens, h, hk, *, rows=None, width=0, causal=True, window=
     p.kv_mode, p.kv_dtype, p.head_dim, p.nheads, p.nheads_k = mode, N.FW_BF16, 128, h, hk
     p.batch, p.seqlen_q, p.seqlen_k = len(rows), sum(rows), sum(lens)
     p.max_seqlen_q, p.causal = max(rows), int(causal)
-    p.window_left, p.window_right = window, -1
+    p.window_left, p.window_right, p.max_seqlen_k = window, -1, longest
     p.k_stride_t = p.v_stride_t = 128
     p.page_size, p.max_pages, p.num_pages = 16, width // 16, 100000
     return p
@@ -219,6 +220,13 @@ def ragged_params(mode, lens, h, hk, *, rows=None, width=0, causal=True, window=
     ("FREE", dict(lens=[900], h=8, hk=2)),
     ("FREE", dict(lens=[1636, 870, 500], h=32, hk=8)),  # 3 workgroups a CU
     ("FREE", dict(lens=[2048, 1000, 5, 700] * 4, h=32, hk=8)),
+    # behind earlier keys: by max_seqlen_k, or without it as if one row had them all
+    ("FREE", dict(rows=[8, 5, 3], lens=[508, 505, 503], h=6, hk=2, longest=508)),
+    ("LARGE", dict(rows=[8, 5, 3], lens=[508, 505, 503], h=6, hk=2)),
+    ("LARGE", dict(rows=[8, 5, 3], lens=[8, 5, 1503], h=6, hk=2, longest=1503)),
+    ("FREE", dict(rows=[900, 100], lens=[900, 100], h=8, hk=2, longest=100000)),
+    ("LARGE", dict(rows=[350] * 32, lens=[350] * 31 + [6350], h=4, hk=4, longest=6350)),
+    ("FREE", dict(rows=[350] * 32, lens=[350] * 31 + [6350], h=32, hk=4, longest=6350)),
     # without the causal mask a row sees twice as many keys
     ("LARGE", dict(lens=[1800] * 8, h=32, hk=8, causal=False)),
     ("FREE", dict(lens=[1800] * 8, h=32, hk=8)),
